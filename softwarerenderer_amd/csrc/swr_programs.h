@@ -91,6 +91,7 @@ template <class L>
 struct ProgCoverage {
     static constexpr int KEY_WORD = REC_KEY;
     static constexpr bool PLANES = false;
+    static constexpr bool LAST_WINS = true;  // any fragment writes the same value
     struct State { bool hit; };
     __device__ static void load(State &s, const RasterArgs &, size_t) { s.hit = false; }
     template <class PX>
@@ -107,13 +108,15 @@ struct ProgCoverage {
 };
 
 // RasterizerTest.cpp:38-48.  Every fragment overwrites the pixel, so only the last one
-// counts: for triangles shade keeps its record (the raster kernel chains nothing, CHAINED)
+// counts: for triangles the raster kernel walks the block's list from its end (LAST_WINS),
+// shade keeps the record of the first fragment met there (the kernel chains nothing, CHAINED)
 // and store chains its colour planes at the pixel (chain_at) and packs them once.
 template <class L>
 struct ProgRGB {
     static constexpr int KEY_WORD = REC_KEY;
     static constexpr bool PLANES = true;
     static constexpr int CHAINED = 0;
+    static constexpr bool LAST_WINS = true;
     struct State { uint32_t c; uint32_t prim; bool hit; };
     __device__ static void load(State &s, const RasterArgs &, size_t)
     {
@@ -490,9 +493,11 @@ template <class L>
 struct ProgTexture {
     static constexpr int KEY_WORD = REC_KEY;
     static constexpr bool PLANES = true;
-    // every fragment overwrites the pixel: shade keeps the last one's record and store
-    // samples once, from the planes chained again at the pixel (chain_at)
+    // every fragment overwrites the pixel: shade keeps the last one's record (the raster
+    // kernel walks the list from its end) and store samples once, from the planes chained
+    // again at the pixel (chain_at)
     static constexpr int CHAINED = 0;
+    static constexpr bool LAST_WINS = true;
     struct State { uint32_t prim; bool hit; };
     __device__ static void load(State &s, const RasterArgs &, size_t)
     {

@@ -59,6 +59,20 @@ struct chained_planes<P, N, decltype((void)P::CHAINED)> {
     static constexpr int value = P::CHAINED < N ? P::CHAINED : N;
 };
 
+// Programs in which a pixel's last fragment alone decides its targets (LAST_WINS): a block
+// walks its list from the end and stops once every pixel has been reached, so its time is
+// bound by the layers above the first covering ones instead of by the list (40,960 large
+// triangles at 640x480, 240 M fragments, Span, RGB: 1987 us in draw order, 64 us this way;
+// one layer, a 1280x720 textured floor: 64 us both ways).
+template <class P, class = void>
+struct last_wins {
+    static constexpr bool value = false;
+};
+template <class P>
+struct last_wins<P, decltype((void)P::LAST_WINS)> {
+    static constexpr bool value = P::LAST_WINS;
+};
+
 // The next work item of a persistent raster workgroup: the first unclaimed item of queue
 // home, home + 1, ... (mod RASTER_QUEUES); queues found empty are not asked again.  `items`
 // items are dealt into the queues as contiguous runs.  NO_ITEM once every queue is empty.
@@ -103,6 +117,7 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
     constexpr int N = L::N;
     constexpr int NS = N > 0 ? N : 1;
     constexpr int NC = chained_planes<Prog, N>::value;  // planes phase A chains
+    constexpr bool LAST = last_wins<Prog>::value;
     // primitives per group: the program's default, or the tuned value
     constexpr int GS = GSX > 0 ? GSX : (N <= 8 ? 8 : (N <= 16 ? 4 : (N <= 32 ? 2 : 1)));
     static_assert(GS >= 1 && GS <= 8, "a group is at most 8 primitives (one per row slot)");
@@ -209,26 +224,29 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                 Prog::load(st, a, o);
             bool drew = false;  // a larger bin's block may keep no primitive: nothing to store
 
-            uint32_t pos = beg;            // next list entry to read
+            // next list entry to read, counted in walking order (LAST: from the list's end)
+            uint32_t pos = 0;
+            const uint32_t num = end - beg;
+            const auto entry = [&](uint32_t k) { return LAST ? end - 1u - k : beg + k; };
             uint32_t head = 0, tail = 0;   // ring of the block's drawn primitives (S > 1)
             for (;;) {
                 int cnt;
                 if (!FILT) {
-                    if (pos >= end)
+                    if (pos >= num)
                         break;
-                    cnt = (int)((end - pos) < (uint32_t)GS ? (end - pos) : (uint32_t)GS);
+                    cnt = (int)((num - pos) < (uint32_t)GS ? (num - pos) : (uint32_t)GS);
                 } else {
-                    while (tail - head < (uint32_t)GS && pos < end) {
+                    while (tail - head < (uint32_t)GS && pos < num) {
                         const uint32_t i = pos + (uint32_t)lane;
                         uint32_t pv = 0;
                         bool keep = false;
-                        if (i < end && MODE == 1) {
-                            pv = a.vals[i];
+                        if (i < num && MODE == 1) {
+                            pv = a.vals[entry(i)];
                             const uint32_t cls = (pv >> (PAIR_CLS4_SHIFT + 2 * bi)) & 3u;
                             keep = cls != 0;
                             pv = (pv & PAIR_CLS4_PRIM_MASK) | cls << 30;
-                        } else if (i < end) {
-                            pv = a.vals[i] & PAIR_PRIM_MASK;
+                        } else if (i < num) {
+                            pv = a.vals[entry(i)] & PAIR_PRIM_MASK;
                             const float *rec = a.prims + (size_t)pv * (size_t)a.stride;
                             const uint32_t flags = __float_as_uint(rec[REC_FLAGS]);
                             if (!SPANS || (flags & FLAG_BLOCK)) {
@@ -265,7 +283,8 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                 const bool act = slot < cnt;
                 uint32_t pv = 0u;
                 if (act)
-                    pv = !FILT ? a.vals[pos + slot] : ring[(head + (uint32_t)slot) & (RING - 1)];
+                    pv = !FILT ? a.vals[entry(pos + (uint32_t)slot)]
+                               : ring[(head + (uint32_t)slot) & (RING - 1)];
                 if (!FILT)
                     pos += (uint32_t)cnt;
                 else
@@ -372,7 +391,8 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                 if (NC == 0)
                     lds_sync();
 
-                // phase B: shade the group's primitives in draw order
+                // phase B: shade the group's primitives in walking order: draw order, or with
+                // LAST the reverse, where only a pixel's first fragment is shaded
 #pragma unroll
                 for (int s2 = 0; s2 < GS; ++s2) {
                     if (s2 < cnt) {
@@ -381,12 +401,18 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                         const uint32_t prim2 =
                             Prog::PLANES ? __builtin_amdgcn_readlane(pv, s2 * 8) & PAIR_PRIM_MASK
                                          : 0u;
-                        if (((m >> lane) & 1ull) && inside)
+                        bool shaded = ((m >> lane) & 1ull) && inside;
+                        if constexpr (LAST)
+                            shaded = shaded && !st.hit;
+                        if (shaded)
                             Prog::shade(st, a, ChainPixel<L, SPANS>{val[s2], prim2}, k2, px,
                                         py);
                     }
                 }
                 lds_sync();
+                if constexpr (LAST)
+                    if (__ballot(inside && !st.hit) == 0ull)
+                        break;  // the rest of the list lies under what is drawn
             }
             if (inside && drew)
                 Prog::template store<ChainPixel<L, SPANS>>(st, a, o, px, py);

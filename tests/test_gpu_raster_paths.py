@@ -1,0 +1,43 @@
+"""The raster kernel's per-program paths at the lengths and edges where they change: lists
+around the group (8) and ring (64) sizes, targets that end inside a block, every bin size,
+against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+from softwarerenderer_amd import scenes
+from helpers import assert_same, run_cpu, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [dict(), dict(raster_waves=1), dict(bin_size=16), dict(bin_size=32, waves_per_bin=2),
+          dict(bin_size=16, raster_queue=1)]
+
+
+def _layers(n, seed, spread):
+    """n triangles over one small screen, near ones smaller, so that blocks have lists of up to
+    n entries, some pixels are covered by all of them and some by none."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-spread, spread, (n, 1, 2))
+    p = c + rng.uniform(0.3, 1.6, (n, 1, 1)) * rng.uniform(-1, 1, (n, 3, 2))
+    v = np.concatenate([np.clip(p, -0.99, 0.99), rng.uniform(-0.9, 0.9, (n, 3, 1)),
+                        rng.random((n, 3, 3))], 2)
+    return scenes.Scene(v.reshape(-1, 6).astype(np.float32), np.arange(3 * n, dtype=np.int32),
+                        np.eye(4, dtype=np.float32), 0, 0)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 64, 65, 200])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+@pytest.mark.parametrize("prog", [O.PS_RGB, O.PS_COVERAGE])
+def test_last_fragment_wins(gpu, cpu_oracle, prog, shape, n):
+    from softwarerenderer_amd import api
+    sc = _layers(n, 100 + n, 0.2 if n > 64 else 0.6)
+    for mode in (O.RASTER_SPAN, O.RASTER_BLOCK, O.RASTER_ADAPTIVE):
+        pipe = O.Pipeline(37, 21, raster_mode=mode, cull_mode=O.CULL_NONE,
+                          vs_program=O.VS_POS_RGB, vs_counts=(1, 3, 0), ps_program=prog,
+                          ps_z=False, ps_w=False, ps_a=3, ps_p=0)
+        r = api.Rasterizer(0)
+        r.setTuning(**SHAPES[shape])
+        assert_same(run_cpu(cpu_oracle, pipe, sc), run_gpu(pipe, sc, rasterizer=r),
+                    f"n={n} mode={mode} {SHAPES[shape]}")
+        r.close()
