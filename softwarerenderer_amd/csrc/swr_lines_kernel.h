@@ -33,15 +33,23 @@ struct VertexPixel {
     uint32_t prim = 0;
 };
 
-// One wave64 per 8x8 tile, lane = pixel: the tile's fragments, 64 at a time, in order.
+// One wave64 per 8x8 tile, lane = pixel: the tile's fragments, 64 at a time.  Lane k loads
+// the round's fragment k into LDS and marks bit k in its pixel's word; every pixel then takes
+// its own fragments, lowest bit first (draw order), so the pixels of a tile shade side by side
+// and a round takes as many steps as its busiest pixel has fragments.  Bound by those steps
+// where many lines meet in a pixel: a 48k-edge wireframe sphere at 1280x720 (its poles) takes
+// 40 us; 64 us with each step's record read from memory, 214 us with the fragments
+// taken one by one, a lane at a time.
 template <template <class> class ProgT, int NZ, int NW, int NA, int NP>
 __global__ void __launch_bounds__(256) k_lines_raster(RasterArgs a)
 {
     using L = Layout<NZ, NW, NA, NP>;
     using Prog = ProgT<L>;
-    const int lane = threadIdx.x & 63;
-    const int tile = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) +
-                                                          (threadIdx.x >> 6)));
+    __shared__ unsigned long long s_mask[4][64];  // per wave: a pixel's fragments of the round
+    constexpr int RW = FR_VAR + L::NA + L::NP, RS = RW | 1;  // odd: records spread over banks
+    __shared__ float s_rec[4][64 * RS];           // the round's fragment records
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int tile = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6)) + wv);
     if (tile >= a.tiles)
         return;
     if (a.status[ST_OVERFLOW] | a.status[ST_ERROR])
@@ -59,21 +67,27 @@ __global__ void __launch_bounds__(256) k_lines_raster(RasterArgs a)
     if (inside)
         Prog::load(st, a, o);
     for (uint32_t c = beg; c < end; c += 64) {
-        const uint32_t n = (end - c) < 64u ? (end - c) : 64u;
-        uint32_t f = 0;
-        int pix = -1;
-        if ((uint32_t)lane < n) {
-            f = a.vals[c + lane];
-            const float *r = a.prims + (size_t)f * (size_t)a.stride;
-            const int fx = (int)__float_as_uint(r[FR_X]), fy = (int)__float_as_uint(r[FR_Y]);
-            pix = (fy - by) * 8 + (fx - bx);
+        s_mask[wv][lane] = 0ull;
+        lds_sync();
+        if (c + (uint32_t)lane < end) {
+            const float *r = a.prims + (size_t)a.vals[c + lane] * (size_t)a.stride;
+            float w[RW];
+#pragma unroll
+            for (int k = 0; k < RW; ++k)
+                w[k] = r[k];
+            const int fx = (int)__float_as_uint(w[FR_X]), fy = (int)__float_as_uint(w[FR_Y]);
+#pragma unroll
+            for (int k = 2; k < RW; ++k)
+                s_rec[wv][lane * RS + k] = w[k];
+            // fragments lie on the target and in this tile: a pixel index below 64
+            atomicOr(&s_mask[wv][((fy - by) * TILE + (fx - bx)) & 63], 1ull << lane);
         }
-        for (uint32_t j = 0; j < n; ++j) {
-            const int pj = __builtin_amdgcn_readlane(pix, (int)j);
-            if (pj != lane || !inside)
-                continue;
-            const uint32_t fj = (uint32_t)__builtin_amdgcn_readlane((int)f, (int)j);
-            const float *r = a.prims + (size_t)fj * (size_t)a.stride;
+        lds_sync();
+        unsigned long long m = s_mask[wv][lane];
+        while (m) {
+            const int j = __builtin_ctzll(m);
+            m &= m - 1ull;
+            const float *r = s_rec[wv] + j * RS;
             VertexPixel<L> p;
             p.zv = r[FR_Z];
             p.wv = r[FR_W];
@@ -85,6 +99,7 @@ __global__ void __launch_bounds__(256) k_lines_raster(RasterArgs a)
                 p.pv[k] = r[FR_VAR + L::NA + k];
             Prog::shade(st, a, p, __float_as_uint(r[kw]), px, py);
         }
+        lds_sync();  // the next round clears the words
     }
     if (inside)
         Prog::template store<VertexPixel<L>>(st, a, o, px, py);

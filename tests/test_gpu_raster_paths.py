@@ -41,3 +41,19 @@ def test_last_fragment_wins(gpu, cpu_oracle, prog, shape, n):
         assert_same(run_cpu(cpu_oracle, pipe, sc), run_gpu(pipe, sc, rasterizer=r),
                     f"n={n} mode={mode} {SHAPES[shape]}")
         r.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 300])
+@pytest.mark.parametrize("prog", [(O.PS_HASH, 3, 2), (O.PS_HASH, 16, 16),
+                                  (O.PS_DEPTH_CHECKER, 3, 2), (O.PS_RGB, 3, 0)])
+def test_fragments_of_a_pixel(gpu, cpu_oracle, prog, n):
+    """n points: half of them in one pixel, the others over a tile that the target cuts."""
+    v = scenes.window_lines(n, 7 + n, 13, 9, margin=0.0)[:n]
+    v["x"][::2], v["y"][::2] = 9.5, 8.25
+    v["x"][1::2] = np.random.default_rng(n).uniform(0, 13, n // 2)
+    v["y"][1::2] = np.random.default_rng(n + 1).uniform(0, 9, n // 2)
+    pipe = O.Pipeline(13, 9, ps_program=prog[0], ps_z=prog[0] != O.PS_RGB,
+                      ps_w=prog[0] != O.PS_RGB, ps_a=prog[1], ps_p=prog[2])
+    idx = np.arange(n, dtype=np.int32)
+    assert_same(run_cpu(cpu_oracle, pipe, vertices=v, indices=idx, prim="point"),
+                run_gpu(pipe, vertices=v, indices=idx, prim="point"), f"n={n} {prog}")
