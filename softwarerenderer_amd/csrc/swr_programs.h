@@ -166,6 +166,7 @@ struct ProgDepthChecker {
     static constexpr int KEY_WORD = REC_KEY;
     static constexpr bool PLANES = true;
     static constexpr int CHAINED = 1;  // z
+    static constexpr bool NEAREST = true;
     struct State { float depth, wr, p0, p1, a0, a1, a2; uint32_t prim; bool hit; };
     __device__ static void load(State &s, const RasterArgs &a, size_t o)
     {
@@ -312,6 +313,7 @@ template <class L>
 struct ProgVisibility {
     static constexpr int KEY_WORD = REC_SRC;
     static constexpr bool PLANES = false;
+    static constexpr bool NEAREST = true;
     struct State { float depth; uint32_t id; bool hit; };
     __device__ static void load(State &s, const RasterArgs &a, size_t o)
     {

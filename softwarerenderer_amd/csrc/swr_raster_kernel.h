@@ -19,15 +19,25 @@
 //
 // Work split.  The chains are independent of draw order, only shading is not.  So the
 // wave takes GS primitives at a time.  Phase A: lane = (slot, row) walks one 8-pixel row
-// of one primitive — 7 adds per parameter produce the row — and the rows go through LDS
-// into pixel-per-lane layout.  Phase B: lane = pixel shades the GS primitives in draw
-// order.
+// of one plane of one primitive — 7 adds produce the row — and the rows go through LDS
+// into pixel-per-lane layout; with fewer than 8 primitives per group (9 planes or more, for
+// the registers' sake) the 8 slots hold several planes of each.  Phase B: lane = pixel shades
+// the GS primitives in draw order.
+//
+// What bounds it: VALU issue (88% of it on dense frames before the steps below).  Per group
+// of 8 primitives the row starts cost 7 DPP additions per chain (14 instructions as additions
+// and selects), programs that only test z take no coverage masks (NaN rows), coverage of
+// every kind is three stepped compares without branches, and a group's record loads leave
+// together.  1080p soup of 1M triangles, Block, 16-pixel bins: 109 -> 88 us; 150k triangles,
+// Adaptive, 1003x701: 87 -> 80 us; 10-plane hash program on 12.7M pairs: 4699 us with half
+// the slots idle, 3237 us with two planes per primitive in them.
 //
 // The kernel is a template over the pixel program, so that programs compiled outside the
 // library (include/swr/pixel_program.h) instantiate it the same way the built-in ones do.
 #pragma once
 
 #include <atomic>
+#include <type_traits>
 
 #include "swr_common.h"
 #include "swr_programs.h"
@@ -72,6 +82,60 @@ template <class P>
 struct last_wins<P, decltype((void)P::LAST_WINS)> {
     static constexpr bool value = P::LAST_WINS;
 };
+
+// Programs that only test z (NEAREST): shade reads nothing but v.z(), under `z < x`, which is
+// false for NaN.  Phase A then writes NaN where the primitive does not cover the pixel, and
+// phase B needs no coverage masks.
+template <class P, class = void>
+struct nearest_only {
+    static constexpr bool value = false;
+};
+template <class P>
+struct nearest_only<P, decltype((void)P::NEAREST)> {
+    static constexpr bool value = P::NEAREST;
+};
+
+// Row starts of a block's chains: lane (slot, row) holds K chains' first-row values v and
+// steps them `row` times by b.  Rows of a slot are two lanes apart (slot_of / row_of below),
+// so a DPP shift by two lanes hands every lane the value of the row above; the lanes of row 0
+// have no source inside their 16 lanes and keep theirs.  After step k lane `row` holds the
+// chain's value after min(row, k) additions: 7 additions per chain instead of 7 additions and
+// 7 selects.  The chains take turns, so a value is read at least two instructions after it is
+// written (the DPP read hazard); the leading s_nop covers the values' producers and a change
+// of the execution mask.  Every lane of a slot is active or none is.
+#define SWR_ROW_STEP(V, B) \
+    "v_add_f32_dpp " V ", " V ", " B " row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+#define SWR_ROW_STEPS(X) X X X X X X X
+__device__ __forceinline__ void row_starts(float (&v)[1], const float (&b)[1])
+{
+    __asm__ volatile("s_nop 4\n\t" SWR_ROW_STEPS(SWR_ROW_STEP("%0", "%1") "s_nop 1\n\t")
+            : "+&v"(v[0])
+            : "v"(b[0]));
+}
+__device__ __forceinline__ void row_starts(float (&v)[2], const float (&b)[2])
+{
+    __asm__ volatile("s_nop 4\n\t" SWR_ROW_STEPS(SWR_ROW_STEP("%0", "%2") SWR_ROW_STEP("%1", "%3")
+                                                     "s_nop 0\n\t")
+                     : "+&v"(v[0]), "+&v"(v[1])
+                     : "v"(b[0]), "v"(b[1]));
+}
+__device__ __forceinline__ void row_starts(float (&v)[3], const float (&b)[3])
+{
+    __asm__ volatile("s_nop 4\n\t" SWR_ROW_STEPS(SWR_ROW_STEP("%0", "%3") SWR_ROW_STEP("%1", "%4")
+                                            SWR_ROW_STEP("%2", "%5"))
+            : "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2])
+            : "v"(b[0]), "v"(b[1]), "v"(b[2]));
+}
+#undef SWR_ROW_STEP
+#undef SWR_ROW_STEPS
+
+// Phase A's lanes: slots 2q and 2q + 1 share 16 lanes, rows two lanes apart.
+__device__ inline int slot_of(int lane) { return ((lane >> 4) << 1) | (lane & 1); }
+__device__ inline int row_of(int lane) { return (lane >> 1) & 7; }
+constexpr int slot_lane(int slot) { return ((slot >> 1) << 4) | (slot & 1); }
+// a slot's 64 row values in LDS, 4 words apart from the next slot's: the two slots of 16 lanes
+// write different banks
+constexpr int SLOT_WORDS = 68;
 
 // The next work item of a persistent raster workgroup: the first unclaimed item of queue
 // home, home + 1, ... (mod RASTER_QUEUES); queues found empty are not asked again.  `items`
@@ -120,12 +184,17 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
     constexpr bool LAST = last_wins<Prog>::value;
     // primitives per group: the program's default, or the tuned value
     constexpr int GS = GSX > 0 ? GSX : (N <= 8 ? 8 : (N <= 16 ? 4 : (N <= 32 ? 2 : 1)));
-    static_assert(GS >= 1 && GS <= 8, "a group is at most 8 primitives (one per row slot)");
-    constexpr int MAXW = 8;  // waves per workgroup: blockDim.x / 64, at most 8
+    static_assert(GS >= 1 && GS <= 8 && (GS & (GS - 1)) == 0, "at most 8 primitives a group");
+    constexpr int PP = 8 / GS;  // planes phase A chains side by side: its 8 slots hold GS
+                                // primitives times PP planes
+    constexpr bool NEAREST = nearest_only<Prog>::value;
+    static_assert(!NEAREST || NC == 1, "a program that only tests z chains z alone");
+    constexpr int MAXW = MODE == 0 ? 8 : 4;  // waves per workgroup: blockDim.x / 64 at most
     constexpr uint32_t RING = 128;  // per-wave ring of a larger bin's drawn primitives
     constexpr int RW = FILT ? MAXW : 1;
-    __shared__ float s_rows[MAXW][GS * 64];
-    __shared__ unsigned long long s_cov[MAXW][GS];
+    constexpr int ROWS = NC > 0 ? 8 * SLOT_WORDS : 4;
+    __shared__ __align__(16) float s_rows[MAXW][ROWS];
+    __shared__ unsigned long long s_cov[NEAREST ? 1 : MAXW][GS];
     __shared__ uint32_t s_ring[RW][RING];
 
     if (a0.fold && blockIdx.x == 0 && threadIdx.x == 0)
@@ -138,9 +207,10 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
         return;
     // phase B: lane = pixel (pi, pj); phase A: lane = (slot, row)
     const int pi = lane & 7, pj = lane >> 3;
-    const int slot = lane >> 3, row = lane & 7;
+    const int lslot = slot_of(lane), row = row_of(lane);
+    const int slot = lslot & (GS - 1), sub = lslot / GS;  // primitive of the group, plane of PP
     float *rows = s_rows[wv];
-    unsigned char *covb = reinterpret_cast<unsigned char *>(s_cov[wv]);
+    unsigned char *covb = reinterpret_cast<unsigned char *>(s_cov[NEAREST ? 0 : wv]);
     uint32_t *ring = s_ring[FILT ? wv : 0];
     const unsigned long long below = (1ull << lane) - 1ull;
 
@@ -289,117 +359,192 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                     pos += (uint32_t)cnt;
                 else
                     head += (uint32_t)cnt;
+                // idle slots (slot >= cnt) read record 0: the loads need no branch
                 const float *__restrict__ rec =
                     a.prims + (size_t)(pv & PAIR_PRIM_MASK) * (size_t)a.stride;
                 const int cls = (int)(pv >> 30);
-                const uint32_t flags = act ? __float_as_uint(rec[REC_FLAGS]) : 0u;
-                const uint32_t key = act ? __float_as_uint(rec[Prog::KEY_WORD]) : 0u;
+                const uint32_t flags = __float_as_uint(rec[REC_FLAGS]);
+                const uint32_t key = __float_as_uint(rec[Prog::KEY_WORD]);
                 const bool blk = !SPANS || (flags & FLAG_BLOCK) != 0;
-
-                // Span: this row's part and [xl, xr) (Rasterizer.h:370-380, 397-407)
-                int xl = 0, xr = 0;
-                bool rowv = false;
-                if (act && !blk)
-                    rowv = span_row_extent(rec, flags, ry, a.sc_minx, a.sc_maxx, xl, xr);
-                const float xs = (float)xl + 0.5f, ys = ryf + 0.5f;
-                const int pre = bx - xl;  // Span: chain steps from xl to the block's first column
-
-                // coverage of this lane's row (8 bits, bit i = column i)
-                uint32_t rowmask = 0;
-                if (act) {
-                    if (blk) {
-                        if (cls == 2) {
-                            rowmask = 0xFFu;
-                        } else {
-                            // the three edges' values at this row's start, then stepped along
-                            // the row together: a pixel is in when all three tests pass
-                            float v[3], ea[3];
-                            bool tie[3];
-#pragma unroll
-                            for (int e = 0; e < 3; ++e) {
-                                ea[e] = rec[REC_EDGE + 3 * e];
-                                const float eb = rec[REC_EDGE + 3 * e + 1],
-                                            ec = rec[REC_EDGE + 3 * e + 2];
-                                tie[e] = (flags >> (1 + e)) & 1u;
-                                float r = ea[e] * xf + eb * yf + ec;
-                                v[e] = r;
-#pragma unroll
-                                for (int k = 1; k < 8; ++k) {
-                                    r = r + eb;
-                                    v[e] = k <= row ? r : v[e];
-                                }
-                            }
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                const bool in = edge_pass(v[0], tie[0]) &&
-                                                edge_pass(v[1], tie[1]) &&
-                                                edge_pass(v[2], tie[2]);
-                                rowmask |= in ? (1u << i) : 0u;
-#pragma unroll
-                                for (int e = 0; e < 3; ++e)
-                                    v[e] = v[e] + ea[e];
-                            }
-                        }
-                    } else if (rowv) {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            rowmask |= (xl <= bx + i && bx + i < xr) ? (1u << i) : 0u;
-                    }
-                    covb[slot * 8 + row] = (unsigned char)rowmask;
+                float zp[3] = {0.0f, 0.0f, 0.0f};
+                if constexpr (NEAREST) {
+                    zp[0] = rec[REC_PARAM];
+                    zp[1] = rec[REC_PARAM + 1];
+                    zp[2] = rec[REC_PARAM + 2];
                 }
 
-                // chained values: phase A row walk, then transpose to pixel-per-lane
+                // Coverage of this lane's row as three functions stepped along its columns: a
+                // pixel is in when each value is at least its limit (edge_pass).  Block: the
+                // edges; a full block, all zero with limit 0; an idle slot or a row without
+                // pixels, an infinite limit.
+                float ev[3] = {0.0f, 0.0f, 0.0f}, ea[3] = {0.0f, 0.0f, 0.0f};
+                float lim[3] = {0.0f, 0.0f, 0.0f};
+                const bool part = act && blk && cls != 2;
+                if (__ballot(part) != 0ull) {
+                    float eb[3];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        ea[e] = rec[REC_EDGE + 3 * e];
+                        eb[e] = rec[REC_EDGE + 3 * e + 1];
+                        ev[e] = ea[e] * xf + eb[e] * yf + rec[REC_EDGE + 3 * e + 2];
+                    }
+                    row_starts(ev, eb);
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        ev[e] = part ? ev[e] : 0.0f;
+                        ea[e] = part ? ea[e] : 0.0f;
+                        lim[e] = part && !((flags >> (1 + e)) & 1u) ? __uint_as_float(1u) : 0.0f;
+                    }
+                }
+                // Span: this row's part and [xl, xr) (Rasterizer.h:370-380, 397-407), as
+                // i - dl >= 0 and dr - 1 - i >= 0
+                int xl = 0, dl = 0;
+                if constexpr (SPANS) {
+                    if (act && !blk) {
+                        int xr = 0;
+                        const bool rowv =
+                            span_row_extent(rec, flags, ry, a.sc_minx, a.sc_maxx, xl, xr);
+                        dl = xl <= bx ? 0 : (xl - bx < 8 ? xl - bx : 8);
+                        const int dr = xr <= bx ? 0 : (xr - bx < 8 ? xr - bx : 8);
+                        ev[0] = -(float)dl;
+                        ea[0] = 1.0f;
+                        ev[1] = (float)(dr - 1);
+                        ea[1] = -1.0f;
+                        lim[2] = rowv ? 0.0f : __builtin_inff();
+                    }
+                }
+                if (!act)
+                    lim[2] = __builtin_inff();
+                const float xs = (float)xl + 0.5f, ys = ryf + 0.5f;
+                const int pre = bx - xl;  // Span: chain steps from xl to the block's first column
+                // whether column i of this lane's row is covered, for i = 0 .. 7 in turn
+                const auto column = [&]() {
+                    const bool in = ev[0] >= lim[0] && ev[1] >= lim[1] && ev[2] >= lim[2];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        ev[e] = ev[e] + ea[e];
+                    return in;
+                };
+                // the first column's value of plane (pa, pb, pc) on this lane's row
+                // (K planes at once: pa, pb, pc; the value replaces pc)
+                const auto first = [&](const auto &pa, const auto &pb, auto &pc) {
+                    constexpr int K = (int)(sizeof(pc) / sizeof(float));
+                    float r[K];
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        r[k] = pa[k] * xf + pb[k] * yf + pc[k];
+                    row_starts(r, pb);
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        if constexpr (SPANS)
+                            if (act && !blk)  // init at xl, then the additions to column 0
+                                r[k] = chain_add(pa[k] * xs + pb[k] * ys + pc[k], pa[k], pre);
+                        pc[k] = r[k];
+                    }
+                };
+
                 float val[GS][NS];
+                float *to = rows + lslot * SLOT_WORDS + row * 8;
+                if constexpr (NEAREST) {
+                    // the z row with NaN where the primitive does not cover the pixel
+                    const float pa[1] = {zp[0]}, pb[1] = {zp[1]};
+                    float z[1] = {zp[2]};
+                    first(pa, pb, z);
 #pragma unroll
-                for (int p = 0; p < NC; ++p) {
-                    float out[8];
-                    if (act) {
-                        const float pa = rec[REC_PARAM + 3 * p], pb = rec[REC_PARAM + 3 * p + 1],
-                                    pc = rec[REC_PARAM + 3 * p + 2];
-                        if (blk) {
-                            // row start: the same chain for every row, kept at this lane's row
-                            float r = pa * xf + pb * yf + pc, r0 = r;
+                    for (int h = 0; h < 2; ++h) {
+                        float q[4];
 #pragma unroll
-                            for (int k = 1; k < 8; ++k) {
-                                r = r + pb;
-                                r0 = k <= row ? r : r0;
-                            }
-                            out[0] = r0;
-#pragma unroll
-                            for (int i = 1; i < 8; ++i)
-                                out[i] = out[i - 1] + pa;
-                        } else {
-                            // init at xl, then the pre additions up to the block's first column
-                            float v = chain_add(pa * xs + pb * ys + pc, pa, pre);
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                out[i] = v;
-                                if (bx + i >= xl)
-                                    v = v + pa;
-                            }
+                        for (int i = 0; i < 4; ++i) {
+                            q[i] = column() ? z[0] : __uint_as_float(0x7FC00000u);
+                            if (!SPANS || 4 * h + i >= dl)
+                                z[0] = z[0] + pa[0];
                         }
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            rows[slot * 64 + row * 8 + i] = out[i];
+                        *reinterpret_cast<float4 *>(to + 4 * h) =
+                            make_float4(q[0], q[1], q[2], q[3]);
                     }
                     lds_sync();
 #pragma unroll
                     for (int s2 = 0; s2 < GS; ++s2)
-                        val[s2][p] = rows[s2 * 64 + pj * 8 + pi];
-                    lds_sync();
+                        val[s2][0] = rows[s2 * SLOT_WORDS + lane];
+                } else {
+                    uint32_t rowmask = 0;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        rowmask |= column() ? (1u << i) : 0u;
+                    if (act && (GS == 8 || sub == 0))
+                        covb[slot * 8 + row] = (unsigned char)rowmask;
+                    // chained values: phase A row walk, then transpose to pixel-per-lane; pass
+                    // t takes planes PP t .. PP t + PP - 1 of every primitive of the group
+                    constexpr int PASSES = (NC + PP - 1) / PP;
+                    const float *pl = rec + REC_PARAM + 3 * sub;
+                    const auto passes = [&](auto kc, int t0) {
+                        constexpr int K = decltype(kc)::value;  // passes whose starts go together
+                        float pa[K], pb[K], v[K];
+#pragma unroll
+                        for (int k = 0; k < K; ++k) {
+                            const int p = PP * (t0 + k);
+                            // lanes past the last plane read it again
+                            const float *q = p + PP <= NC || sub < NC - p
+                                                 ? pl + 3 * p
+                                                 : rec + REC_PARAM + 3 * (NC - 1);
+                            pa[k] = q[0];
+                            pb[k] = q[1];
+                            v[k] = q[2];
+                        }
+                        first(pa, pb, v);
+#pragma unroll
+                        for (int k = 0; k < K; ++k) {
+                            float out[8];
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) {
+                                out[i] = v[k];
+                                if (!SPANS || i >= dl)
+                                    v[k] = v[k] + pa[k];
+                            }
+                            *reinterpret_cast<float4 *>(to) =
+                                make_float4(out[0], out[1], out[2], out[3]);
+                            *reinterpret_cast<float4 *>(to + 4) =
+                                make_float4(out[4], out[5], out[6], out[7]);
+                            lds_sync();
+#pragma unroll
+                            for (int u = 0; u < PP; ++u) {
+                                const int p = PP * (t0 + k) + u;
+                                if (p < NC)
+#pragma unroll
+                                    for (int s2 = 0; s2 < GS; ++s2)
+                                        val[s2][p] = rows[(u * GS + s2) * SLOT_WORDS + lane];
+                            }
+                            lds_sync();
+                        }
+                    };
+#pragma unroll
+                    for (int t = 0; t + 3 <= PASSES; t += 3)
+                        passes(std::integral_constant<int, 3>{}, t);
+                    if constexpr (PASSES % 3 == 2)
+                        passes(std::integral_constant<int, 2>{}, PASSES - 2);
+                    else if constexpr (PASSES % 3 == 1)
+                        passes(std::integral_constant<int, 1>{}, PASSES - 1);
+                    if (NC == 0)
+                        lds_sync();
                 }
-                if (NC == 0)
-                    lds_sync();
 
                 // phase B: shade the group's primitives in walking order: draw order, or with
                 // LAST the reverse, where only a pixel's first fragment is shaded
 #pragma unroll
                 for (int s2 = 0; s2 < GS; ++s2) {
-                    if (s2 < cnt) {
-                        const unsigned long long m = s_cov[wv][s2];
-                        const uint32_t k2 = __builtin_amdgcn_readlane(key, s2 * 8);
+                    if constexpr (NEAREST) {  // slots beyond cnt hold NaN
+                        const uint32_t k2 = __builtin_amdgcn_readlane(key, slot_lane(s2));
                         const uint32_t prim2 =
-                            Prog::PLANES ? __builtin_amdgcn_readlane(pv, s2 * 8) & PAIR_PRIM_MASK
+                            Prog::PLANES ? __builtin_amdgcn_readlane(pv, slot_lane(s2)) &
+                                               PAIR_PRIM_MASK
+                                         : 0u;
+                        Prog::shade(st, a, ChainPixel<L, SPANS>{val[s2], prim2}, k2, px, py);
+                    } else if (s2 < cnt) {
+                        const unsigned long long m = s_cov[wv][s2];
+                        const uint32_t k2 = __builtin_amdgcn_readlane(key, slot_lane(s2));
+                        const uint32_t prim2 =
+                            Prog::PLANES ? __builtin_amdgcn_readlane(pv, slot_lane(s2)) &
+                                               PAIR_PRIM_MASK
                                          : 0u;
                         bool shaded = ((m >> lane) & 1ull) && inside;
                         if constexpr (LAST)

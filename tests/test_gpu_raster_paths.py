@@ -57,3 +57,32 @@ def test_fragments_of_a_pixel(gpu, cpu_oracle, prog, n):
     idx = np.arange(n, dtype=np.int32)
     assert_same(run_cpu(cpu_oracle, pipe, vertices=v, indices=idx, prim="point"),
                 run_gpu(pipe, vertices=v, indices=idx, prim="point"), f"n={n} {prog}")
+
+
+GROUPS = SHAPES + [dict(raster_group=1), dict(raster_group=2, bin_size=16),
+                   dict(raster_group=4, bin_size=32)]
+
+
+@pytest.mark.parametrize("n", [1, 3, 8, 9, 70])
+@pytest.mark.parametrize("shape", range(len(GROUPS)))
+@pytest.mark.parametrize("prog", [(O.PS_HASH, 4, 4), (O.PS_HASH, 16, 16), (O.PS_HASH, 0, 0),
+                                  (O.PS_DEPTH_CHECKER, 3, 2), (O.PS_VISIBILITY, 0, 0)])
+def test_chained_planes(gpu, cpu_oracle, prog, shape, n):
+    """Every interpolant of every fragment (hash), and the nearest fragment, for lists of n
+    primitives in blocks that the target's right and lower edges cut."""
+    from softwarerenderer_amd import api
+    rng = np.random.default_rng(n)
+    lay = _layers(n, 300 + n, 0.5)
+    w = rng.uniform(0.5, 2.0, (3 * n, 1))
+    na, np_ = max(prog[1], 1), max(prog[2], 1)
+    v = np.concatenate([lay.vertices[:, :3] * w, w, rng.random((3 * n, na + np_))], 1)
+    sc = scenes.Scene(v.astype(np.float32), lay.indices, np.eye(4, dtype=np.float32), 0, 0)
+    for mode in (O.RASTER_SPAN, O.RASTER_BLOCK, O.RASTER_ADAPTIVE):
+        pipe = O.Pipeline(37, 21, raster_mode=mode, cull_mode=O.CULL_NONE, vs_program=O.VS_RAW,
+                          vs_counts=(1, na, np_), ps_program=prog[0], ps_z=True,
+                          ps_w=prog[0] != O.PS_VISIBILITY, ps_a=prog[1], ps_p=prog[2])
+        r = api.Rasterizer(0)
+        r.setTuning(**GROUPS[shape])
+        assert_same(run_cpu(cpu_oracle, pipe, sc), run_gpu(pipe, sc, rasterizer=r),
+                    f"n={n} mode={mode} {GROUPS[shape]} {prog}")
+        r.close()
