@@ -30,13 +30,13 @@
 // of every pair's decision; pairs that need the silhouette walk go to a queue),
 // k_diff_march (one lane per queued pair: the walk, the stored decision, per-tile flags),
 // k_diff_blend (only tiles with an active pair: the antialiasing added to the image).
-// Backward: k_diff_backward<INTERIOR> (every pixel: its own triangle's interpolation under
-// dL/dimage) and k_diff_backward<EDGES> (flagged tiles only: what the antialiasing adds),
+// Backward: k_diff_bwd_interior (every pixel: its own triangle's interpolation under
+// dL/dimage) and k_diff_bwd_edges (the active pairs: what the antialiasing adds),
 // both reading the stored decisions; gradients reach the vertex attributes through b_i,
 // the clip coordinates through D_i (barycentrics) and through t (the silhouette crossing),
 // accumulated per tile in LDS and flushed with float atomics.  A backward whose buffers are
 // not those of the last forward on the context takes decisions again itself
-// (k_diff_backward<ALL>).  The walk is queued because few pairs need it (about 1% on a
+// (k_diff_backward).  The walk is queued because few pairs need it (about 1% on a
 // 41k-vertex sphere at 512 x 512) and a wave that holds one waits on its chain of dependent
 // loads with all 64 lanes.
 //
@@ -80,10 +80,11 @@ struct DiffArgs {
                        // bit 1 some pair to the right of its last column, bit 2 some pair
                        // below its last row
     // per (view, tile) b: the pairs that need the silhouette walk (pair index 2 * pixel +
-    // dir) at queue[b * 512 ..) with qcnt[b] entries, and the pixels with an active pair (the
-    // blend pass lists them) at elist[b * 256 ..) with ecnt[b] entries
+    // dir) at queue[b * 512 ..) with qcnt[b] entries, and the active ones of the tile's own
+    // pairs (the blend pass lists them) at elist[b * 512 ..) with ecnt[b] entries
     uint32_t *queue, *qcnt;
     uint32_t *elist, *ecnt;
+    int row_keys;  // 1: clip rows fit the int keys of the edge backward's table
     int pairs;     // 0: evaluate, 1: evaluate and store, 2: load the stored decisions
     // several meshes (null for one): per view, the clip row of global vertex g is
     // vrow[view] + g and visibility id k names triangle vtri[view].x + k - 1 (k <= .y);
@@ -501,13 +502,10 @@ __device__ inline void pixel_color(const DiffArgs &d, int view, size_t i, int px
 // table in LDS keyed by vertex, flushed to global memory once per distinct vertex.  The
 // pixels of a tile touch a few dozen vertices, so this replaces most global float atomics
 // (which serialise on shared vertices) by LDS atomics.  A vertex that finds no slot after
-// `probes` probes goes straight to global memory.  Slots are never freed, so a vertex that
+// ACC_PROBES probes goes straight to global memory.  Slots are never freed, so a vertex that
 // got a slot is found again within the same probes.
 constexpr int ACC_SLOTS = 256;   // power of two
 constexpr int ACC_PROBES = 32;   // one 16x16 tile: a few dozen vertices, the table never fills
-// the edge backward's table serves a group of 64 tiles, whose silhouette pixels can touch
-// more vertices than it holds: a full table then costs every new vertex all its probes
-constexpr int ACC_PROBES_SPARSE = 8;
 constexpr int ACC_VALS = 8;      // at most: clip x, y, w, attributes 0..4
 // values per slot with C attribute channels: clip x, y, w and the C attributes
 template <int C> constexpr int acc_vals() { return 3 + C; }
@@ -521,16 +519,13 @@ __device__ inline int acc_copy() { return (int)((threadIdx.x & 1u) | ((threadIdx
 struct VertexAcc {
     int *key;
     float *val;
-    int probes;
 };
 
 __device__ inline int acc_slot(const VertexAcc &A, int v)
 {
-    if (!A.key)
-        return -1;  // no table: straight to global memory
     const unsigned h = ((unsigned)v * 2654435761u) >> 24;  // 8 bits: ACC_SLOTS
 #pragma unroll 1
-    for (int probe = 0; probe < A.probes; ++probe) {
+    for (int probe = 0; probe < ACC_PROBES; ++probe) {
         const int sl = (int)((h + (unsigned)probe) & (ACC_SLOTS - 1));
         const int k = __atomic_load_n(&A.key[sl], __ATOMIC_RELAXED);
         if (k == v)
@@ -866,24 +861,27 @@ __device__ inline Pair unpack_pair(const PairLds &x, bool swap, bool horiz)
 
 
 
-// A workgroup's share of per-tile segments: TILES_PER_GROUP consecutive tiles, their
-// lengths scanned into s_off (s_off[k] = entries before tile k, s_off[64] = all), so the
-// workgroup's threads take the entries densely, one each.
+// A workgroup's share of per-tile segments: TILES consecutive tiles, their lengths scanned
+// into s_off (s_off[k] = entries before tile k, s_off[TILES] = all), so the workgroup's threads
+// take the entries densely, one each.
 constexpr int TILES_PER_GROUP = 64;
 
+template <int TILES>
 __device__ inline void group_segments(const uint32_t *cnt, uint32_t tiles, uint32_t t0,
                                       uint32_t *s_off)
 {
+    static_assert(TILES <= 64, "a tile per lane of the first wave");
     if (threadIdx.x < 64) {
         const uint32_t lane = threadIdx.x;
-        uint32_t v = t0 + lane < tiles ? cnt[t0 + lane] : 0u;
+        uint32_t v = lane < TILES && t0 + lane < tiles ? cnt[t0 + lane] : 0u;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const uint32_t u = __shfl_up(v, o, 64);
             if ((int)lane >= o)
                 v += u;
         }
-        s_off[lane + 1] = v;
+        if (lane < TILES)
+            s_off[lane + 1] = v;
         if (lane == 0)
             s_off[0] = 0;
     }
@@ -891,9 +889,10 @@ __device__ inline void group_segments(const uint32_t *cnt, uint32_t tiles, uint3
 }
 
 // The tile (within the group) of entry j: the largest k with s_off[k] <= j.
+template <int TILES>
 __device__ inline uint32_t group_tile(const uint32_t *s_off, uint32_t j)
 {
-    uint32_t lo = 0, hi = TILES_PER_GROUP;
+    uint32_t lo = 0, hi = TILES;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
         if (s_off[mid] <= j)
@@ -914,11 +913,11 @@ __global__ void __launch_bounds__(MARCH_THREADS) k_diff_march(DiffArgs d)
 {
     __shared__ uint32_t s_off[TILES_PER_GROUP + 1];
     const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * TILES_PER_GROUP;
-    group_segments(d.qcnt, tiles, t0, s_off);
+    group_segments<TILES_PER_GROUP>(d.qcnt, tiles, t0, s_off);
     const uint32_t n = s_off[TILES_PER_GROUP];
     const size_t HW = (size_t)d.W * d.H;
     for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) {
-        const uint32_t t = group_tile(s_off, j);
+        const uint32_t t = group_tile<TILES_PER_GROUP>(s_off, j);
         const uint32_t k = d.queue[(size_t)(t0 + t) * 512 + (j - s_off[t])];
         const size_t i = k >> 1;
         const int dir = (int)(k & 1u);
@@ -997,28 +996,21 @@ __device__ inline void tile_pairs(const DiffArgs &d, const PixelIdx &pi, bool va
         v[lx] = eval_packed(d, view, px, py - 1, px, py);
 }
 
+// This thread's own pair dir (0: to its right, 1: below) in the tile's table.
+__device__ inline const PairLds &tile_own(const PairLds *h, const PairLds *v, int dir)
+{
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
+    return dir == 0 ? h[ly * 17 + lx + 1] : v[(ly + 1) * 16 + lx];
+}
+
 // The pair between this thread's pixel and neighbour k (0 right, 1 left, 2 below, 3 above).
 __device__ inline Pair tile_pair(const PairLds *h, const PairLds *v, int k);
 
-// Where a pixel's four pairs come from: the workgroup's LDS table, or the stored decisions.
+// A pixel's four pairs from the workgroup's LDS table.
 struct TilePairs {
     const PairLds *h, *v;
     __device__ Pair get(int k) const { return tile_pair(h, v, k); }
 };
-struct StoredPairs {
-    PairLds p[4];  // right, left, below, above, each seen from its left / upper pixel
-    __device__ StoredPairs(const DiffArgs &d, size_t i, int px, int py)
-    {
-        PairLds none;
-        none.flags = 0;
-        p[0] = px + 1 < d.W ? load_pair(d, 2 * i) : none;
-        p[1] = px > 0 ? load_pair(d, 2 * (i - 1)) : none;
-        p[2] = py + 1 < d.H ? load_pair(d, 2 * i + 1) : none;
-        p[3] = py > 0 ? load_pair(d, 2 * (i - d.W) + 1) : none;
-    }
-    __device__ Pair get(int k) const { return unpack_pair(p[k], k == 1 || k == 3, k < 2); }
-};
-
 __device__ inline Pair tile_pair(const PairLds *h, const PairLds *v, int k)
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
@@ -1048,14 +1040,12 @@ __global__ void __launch_bounds__(256) k_diff_blend(DiffArgs d)
     const bool valid = pixel_of_thread(d, pi);
     tile_pairs<true>(d, pi, valid, s_h, s_v);
     __syncthreads();
-    // the backward pass's antialiasing work is per pixel with an active pair: list them
-    bool any = false;
-    for (int k = 0; k < 4 && valid; ++k) {
-        int qx, qy;
-        any = any || (neighbour(d, pi.px, pi.py, k, qx, qy) && tile_pair(s_h, s_v, k).active);
-    }
+    // the backward pass's antialiasing work is per active pair: list the pixels' own two
     const int b = xcd_order(blockIdx.x, gridDim.x);
-    tile_append2(d.elist + (size_t)b * 256, d.ecnt + b, any, any ? (uint32_t)pi.i : 0u, false, 0u);
+    const bool right = valid && (tile_own(s_h, s_v, 0).flags & 1),
+               down = valid && (tile_own(s_h, s_v, 1).flags & 1);
+    const uint32_t k0 = right || down ? (uint32_t)(2 * pi.i) : 0u;
+    tile_append2(d.elist + (size_t)b * 512, d.ecnt + b, right, k0, down, k0 + 1u);
     if (!valid)
         return;
     const size_t i = pi.i;
@@ -1104,12 +1094,8 @@ __device__ inline void scatter_window_grad(const DiffArgs &d, const VertexAcc &A
              (float)((-gx * sx * h.x + gy * sy * h.y) * iw * iw));
 }
 
-// Which part of a pixel's gradient backward_pixel computes: everything, only the
-// interpolation of its own triangle under dL/dimage, or only what the antialiasing adds
-// (the interpolation backward is linear in the colour gradient, so the two parts add up).
-enum BwdPart { BWD_ALL, BWD_INTERIOR, BWD_EDGES };
-
-template <int C, int PART, class PS>
+// A pixel's whole gradient: the interpolation of its own triangle and the antialiasing.
+template <int C, class PS>
 __device__ inline void backward_pixel(const DiffArgs &d, const VertexAcc &A, const PixelIdx &pi,
                                       const PS &pairs)
 {
@@ -1120,15 +1106,13 @@ __device__ inline void backward_pixel(const DiffArgs &d, const VertexAcc &A, con
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         gp[c] = grad_image(d, i, C, c);
-        gc[c] = PART == BWD_EDGES ? 0.0 : gp[c];
+        gc[c] = gp[c];
         cp[c] = 0.0;
     }
-    if (PART != BWD_INTERIOR)
-        pixel_color<C>(d, view, i, px, py, cp);
-    bool touched = PART != BWD_EDGES;
+    pixel_color<C>(d, view, i, px, py, cp);
 
     // antialiasing: colour gradients (gather) and silhouette crossings (scatter)
-    for (int k = 0; k < 4 && PART != BWD_INTERIOR; ++k) {
+    for (int k = 0; k < 4; ++k) {
         int qx, qy;
         if (!neighbour(d, px, py, k, qx, qy))
             continue;
@@ -1145,7 +1129,6 @@ __device__ inline void backward_pixel(const DiffArgs &d, const VertexAcc &A, con
 #pragma unroll
                 for (int c = 0; c < C; ++c)
                     gc[c] += w * grad_image(d, iq, C, c);
-                touched = true;
             }
             continue;
         }
@@ -1178,7 +1161,6 @@ __device__ inline void backward_pixel(const DiffArgs &d, const VertexAcc &A, con
             gc[c] -= w * gp[c];
             dot += gp[c] * (src[c] - cp[c]);
         }
-        touched = true;
         const double dldt = pv.a * (t_low ? -dot : dot) + dedt, dlda = wt * dot;
         scatter_window_grad<C>(d, A, view, pr.vj, dldt * pv.tj.x + dlda * pv.aj.x,
                             dldt * pv.tj.y + dlda * pv.aj.y);
@@ -1187,8 +1169,6 @@ __device__ inline void backward_pixel(const DiffArgs &d, const VertexAcc &A, con
     }
 
     // barycentric interpolation of the pixel's own triangle
-    if (!touched)
-        return;
     const uint32_t id = d.ids[i];
     Bary B;
     const int tri = id_tri(d, view, id);
@@ -1214,9 +1194,9 @@ __global__ void __launch_bounds__(256) k_diff_backward(DiffArgs d)
     const bool valid = pixel_of_thread(d, pi);
     tile_pairs<false>(d, pi, valid, s_h, s_v);
     __syncthreads();
-    const VertexAcc A{s_key, s_val, ACC_PROBES};
+    const VertexAcc A{s_key, s_val};
     if (valid)  // every thread reaches the barrier below
-        backward_pixel<C, BWD_ALL>(d, A, pi, TilePairs{s_h, s_v});
+        backward_pixel<C>(d, A, pi, TilePairs{s_h, s_v});
     __syncthreads();
     acc_flush<C>(d, A, pi.view);
 }
@@ -1303,56 +1283,222 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
     SWR_MERGE(4)
 #undef SWR_MERGE
     __syncthreads();
-    const VertexAcc A{s_key, s_val, ACC_PROBES};
+    const VertexAcc A{s_key, s_val};
     if (keep)
         acc_triangle<C>(d, A, pi.view, vid, g);
     __syncthreads();
     acc_flush<C>(d, A, pi.view);
 }
 
-// What the antialiasing adds to the gradients, for the pixels the blend pass listed (one
-// lane each; the decisions come from the forward's store).  Vertex gradients are summed in
-// an LDS table keyed by vertex when the group's tiles lie in one view (silhouette pixels of
-// a ridge share its vertices), else they go straight to global memory.
+// ---- what the antialiasing adds to the gradients ---------------------------------------------
+// One lane per active pair (the blend pass listed them; the decisions come from the forward's
+// store).  A pair blends one pixel B with a source colour: when the crossing lies in the front
+// pixel's half, B is the front pixel and the source the other pixel's colour, else B is the
+// other pixel and the source the silhouette triangle's colour at the crossing.  Either way the
+// source is a triangle's interpolation along a ray, so all lanes run the same code: B's and
+// the source's interpolation, forward and backward, and the crossing's derivatives, whose
+// gradients join those of the triangle that owns the edge.  Bound by the latency of that chain
+// (dependent loads, fp64 divisions), so it is kept short: with a lane per pixel and its four
+// pairs in turn, three divergent cases each, one 256x256 view took 79 us and 64 views of
+// 512x512 553 us (beside the interior kernel); now 30 and 171 us.
+//
+// Gradients are summed in an LDS table keyed by clip row (neighbouring silhouette pairs share
+// vertices), one wave per table; a row that finds no slot goes to global memory.
+constexpr int EDGE_TILES = 16;   // tiles per workgroup of one wave
+constexpr int EDGE_SLOTS = 128;  // power of two
+constexpr int EDGE_PROBES = 8;
+constexpr int EDGE_COPIES = 2;   // of each value, picked by lane parity
+
 template <int C>
-__global__ void __launch_bounds__(256) k_diff_bwd_edges(DiffArgs d)
+struct EdgeAcc {
+    static constexpr int STRIDE = (3 + C) * EDGE_COPIES + 1;  // odd: slots spread over the banks
+    int key[EDGE_SLOTS];
+    float val[EDGE_SLOTS * STRIDE];
+};
+
+// Adds {clip x, y, w, attributes} to row `row`; attr = false: the clip part only.
+template <int C>
+__device__ inline void edge_add(const DiffArgs &d, EdgeAcc<C> &A, size_t row,
+                                const float (&g)[3 + C], bool attr)
 {
-    __shared__ uint32_t s_off[TILES_PER_GROUP + 1];
-    __shared__ int s_key[ACC_SLOTS];
-    __shared__ __align__(16) float s_val[ACC_SLOTS * acc_vals<C>() * ACC_COPIES];
-    const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * TILES_PER_GROUP;
-    group_segments(d.ecnt, tiles, t0, s_off);
-    const uint32_t n = s_off[TILES_PER_GROUP];
-    if (n == 0)
-        return;  // n is the same for every thread of the group
-    const uint32_t t_last = (t0 + TILES_PER_GROUP < tiles ? t0 + TILES_PER_GROUP : tiles) - 1;
-    const int view0 = (int)(t0 / (uint32_t)d.tiles_per_view);
-    const bool one_view = (uint32_t)view0 == t_last / (uint32_t)d.tiles_per_view;
-    if (one_view) {
-        for (int sl = threadIdx.x; sl < ACC_SLOTS; sl += blockDim.x)
-            s_key[sl] = -1;
-        for (int k = threadIdx.x; k < ACC_SLOTS * acc_vals<C>() * ACC_COPIES / 4; k += blockDim.x)
-            reinterpret_cast<float4 *>(s_val)[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        __syncthreads();
+    int slot = -1;
+    if (d.row_keys) {
+        const unsigned h = ((unsigned)row * 2654435761u) >> 25;  // 7 bits: EDGE_SLOTS
+#pragma unroll 1
+        for (int probe = 0; probe < EDGE_PROBES && slot < 0; ++probe) {
+            const int sl = (int)((h + (unsigned)probe) & (EDGE_SLOTS - 1));
+            const int old = atomicCAS(&A.key[sl], -1, (int)row);
+            if (old == -1 || old == (int)row)
+                slot = sl;
+        }
     }
+    if (slot >= 0) {
+        float *x = &A.val[slot * EdgeAcc<C>::STRIDE + (int)(threadIdx.x & (EDGE_COPIES - 1))];
+#pragma unroll
+        for (int k = 0; k < 3 + C; ++k)
+            if (k < 3 || attr)
+                atomicAdd(x + k * EDGE_COPIES, g[k]);
+        return;
+    }
+    atomicAdd(d.gclip + row * 4 + 0, g[0]);
+    atomicAdd(d.gclip + row * 4 + 1, g[1]);
+    atomicAdd(d.gclip + row * 4 + 3, g[2]);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        if (attr)
+            atomicAdd(d.gattr + row * C + c, g[3 + c]);
+}
+
+template <int C>
+__device__ inline void edge_flush(const DiffArgs &d, const EdgeAcc<C> &A)
+{
+    static_assert(EDGE_COPIES == 2, "the flush adds two copies");
+    for (int sl = threadIdx.x; sl < EDGE_SLOTS; sl += 64) {
+        const int row = A.key[sl];
+        if (row < 0)
+            continue;
+        const float *x = &A.val[sl * EdgeAcc<C>::STRIDE];
+#pragma unroll
+        for (int k = 0; k < 3 + C; ++k) {
+            const float v = x[k * EDGE_COPIES] + x[k * EDGE_COPIES + 1];
+            float *to = k < 3 ? d.gclip + (size_t)row * 4 + (k == 2 ? 3 : k)
+                              : d.gattr + (size_t)row * C + (k - 3);
+            if (v != 0.0f)
+                atomicAdd(to, v);
+        }
+    }
+}
+
+// d(window x, y) of a clip-space vertex -> d(clip x, y, w).
+__device__ inline void window_grad(const DiffArgs &d, const H3 &h, double gx, double gy,
+                                   float (&out)[3])
+{
+    const double iw = 1.0 / h.w, sx = 0.5 * d.W, sy = 0.5 * d.H;
+    out[0] = (float)(gx * sx * iw);
+    out[1] = (float)(-gy * sy * iw);
+    out[2] = (float)((-gx * sx * h.x + gy * sy * h.y) * iw * iw);
+}
+
+template <int C>
+__device__ inline void backward_pair(const DiffArgs &d, EdgeAcc<C> &A, uint32_t k)
+{
     const size_t HW = (size_t)d.W * d.H;
-    const VertexAcc A = one_view ? VertexAcc{s_key, s_val, ACC_PROBES_SPARSE}
-                                   : VertexAcc{nullptr, nullptr, 0};
-    for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) {
-        const uint32_t t = group_tile(s_off, j);
-        PixelIdx pi;
-        pi.i = d.elist[(size_t)(t0 + t) * 256 + (j - s_off[t])];
-        pi.view = (int)(pi.i / HW);
-        const size_t rem = pi.i - (size_t)pi.view * HW;
-        pi.py = (int)(rem / (size_t)d.W);
-        pi.px = (int)(rem - (size_t)pi.py * d.W);
-        pi.tile = 0;
-        backward_pixel<C, BWD_EDGES>(d, A, pi, StoredPairs(d, pi.i, pi.px, pi.py));
+    const size_t i = k >> 1;
+    const int dir = (int)(k & 1u);
+    const int view = (int)(i / HW);
+    const size_t rem = i - (size_t)view * HW;
+    const int py = (int)(rem / (size_t)d.W), px = (int)(rem - (size_t)py * d.W);
+    const int qx = px + (dir == 0), qy = py + (dir == 1);
+    const PairLds x = load_pair(d, k);
+    const Pair pr = unpack_pair(x, false, dir == 0);
+    const size_t iq = i + (dir == 0 ? (size_t)1 : (size_t)d.W);
+    const size_t ib = pr.p_blended ? i : iq, io = pr.p_blended ? iq : i;
+    const int bx = pr.p_blended ? px : qx, by = pr.p_blended ? py : qy;
+    const int ox = pr.p_blended ? qx : px, oy = pr.p_blended ? qy : py;
+    const bool t_low = pr.tf < 0.5f;  // B is the front pixel
+
+    const PairVal pv = pair_val(d, view, pr, px, py, qx, qy);
+    const double wt = t_low ? 0.5 - pv.t : pv.t - 0.5, w = pv.a * wt;
+    double g[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        g[c] = grad_image(d, ib, C, c);
+
+    // the source: the other pixel's triangle at its centre, or the silhouette's at the crossing
+    Bary S, B;
+    H3 drdt;
+    const int tri_s = t_low ? id_tri(d, view, d.ids[io]) : pr.tri;
+    H3 ray = crossing_ray(d, pr, pv.t, px, py, qx, qy, drdt);
+    if (t_low)
+        ray = pixel_ray(d, ox, oy);
+    const bool has_s = tri_s >= 0 && bary_at_ray(d, view, tri_s, ray, S);
+    if (!t_low && !has_s)
+        return;  // the blend skipped it too
+    const int tri_b = id_tri(d, view, d.ids[ib]);
+    const bool has_b = tri_b >= 0 && bary_at(d, view, tri_b, bx, by, B);
+    double src[C], cp[C], de[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        src[c] = cp[c] = de[c] = 0.0;
+    if (has_s) {
+        bary_color<C>(d, S, src);
+        if (!t_low)
+            bary_color_dr<C>(d, S, drdt, de);
     }
-    if (one_view) {
-        __syncthreads();
-        acc_flush<C>(d, A, view0);
+    if (has_b)
+        bary_color<C>(d, B, cp);
+    double dot = 0.0, dedt = 0.0, gs[C], gb[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        // a pixel's colour is an fp32 image value
+        const double s = t_low ? (double)(float)src[c] : src[c];
+        dot += g[c] * (s - (double)(float)cp[c]);
+        gs[c] = w * g[c];
+        gb[c] = -gs[c];
+        dedt += gs[c] * de[c];
     }
+    // the crossing: its edge's vertices j and k
+    const double dldt = pv.a * (t_low ? -dot : dot) + dedt, dlda = wt * dot;
+    float wj[3], wk[3];
+    window_grad(d, load_h(d, view, pr.vj), dldt * pv.tj.x + dlda * pv.aj.x,
+                dldt * pv.tj.y + dlda * pv.aj.y, wj);
+    window_grad(d, load_h(d, view, pr.vk), dldt * pv.tk.x + dlda * pv.ak.x,
+                dldt * pv.tk.y + dlda * pv.ak.y, wk);
+    // the triangle that owns the edge is the source's, or mostly the front pixel's own
+    const bool in_s = has_s && tri_s == pr.tri, in_b = !in_s && has_b && tri_b == pr.tri;
+    const auto triangle = [&](const Bary &T, const double *gc, bool own) {
+        float out[3][3 + C];
+        bary_grads<C>(d, T, gc, out);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            if (own) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n)
+                    out[m][n] += T.v[m] == pr.vj ? wj[n] : (T.v[m] == pr.vk ? wk[n] : 0.0f);
+            }
+            edge_add<C>(d, A, crow(d, view, T.v[m]), out[m], true);
+        }
+    };
+    if (has_s)
+        triangle(S, gs, in_s);
+    if (has_b)
+        triangle(B, gb, in_b);
+    if (!in_s && !in_b) {
+        float out[3 + C];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            out[3 + c] = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+                out[n] = v == 0 ? wj[n] : wk[n];
+            edge_add<C>(d, A, crow(d, view, v == 0 ? pr.vj : pr.vk), out, false);
+        }
+    }
+}
+
+template <int C>
+__global__ void __launch_bounds__(64) k_diff_bwd_edges(DiffArgs d)
+{
+    __shared__ EdgeAcc<C> A;
+    __shared__ uint32_t s_off[EDGE_TILES + 1];
+    const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * EDGE_TILES;
+    group_segments<EDGE_TILES>(d.ecnt, tiles, t0, s_off);
+    const uint32_t n = s_off[EDGE_TILES];
+    if (n == 0)
+        return;
+    for (int sl = threadIdx.x; sl < EDGE_SLOTS; sl += 64)
+        A.key[sl] = -1;
+    for (int k = threadIdx.x; k < EDGE_SLOTS * EdgeAcc<C>::STRIDE; k += 64)
+        A.val[k] = 0.0f;
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < n; j += 64) {
+        const uint32_t t = group_tile<EDGE_TILES>(s_off, j);
+        backward_pair<C>(d, A, d.elist[(size_t)(t0 + t) * 512 + (j - s_off[t])]);
+    }
+    __syncthreads();
+    edge_flush<C>(d, A);
 }
 
 // grad_attributes += sum over the views that see the vertex (in view order) of the
@@ -1421,7 +1567,8 @@ static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const
                     return e;
                 se = side.s;
             }
-            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3(groups), dim3(256), 0, se, d);
+            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3((blocks + EDGE_TILES - 1) / EDGE_TILES),
+                               dim3(64), 0, se, d);
             hipLaunchKernelGGL(k_diff_bwd_interior<C>, dim3(blocks), dim3(256), 0, s, d);
             if (fork) {
                 hipError_t e = hipEventRecord(side.join, side.s);
@@ -1550,13 +1697,14 @@ static int diff_run(swr_context *c, const swr_diff_desc *dd, const float *gimage
     // The forward stores its pair decisions; a backward over the same buffers and sizes
     // reuses them instead of walking the silhouettes again.
     // layout: flags [2 px] u8, data [2 px] int2, per tile: flags, queue and list lengths
-    // u32, queue [tiles][512] u32, list [tiles][256] u32
+    // u32, queue [tiles][512] u32, list [tiles][512] u32
     const size_t tiles = (size_t)d.tiles_per_view * d.V, off_f = 0,
                  off_d = (off_f + px * 2 + 15) & ~(size_t)15, off_t = off_d + px * 2 * sizeof(int2),
                  off_q = (off_t + tiles * 12 + 15) & ~(size_t)15, off_e = off_q + tiles * 512 * 4;
+    d.row_keys = rows <= 0x7FFFFFFFull ? 1 : 0;
     if (px * 2 > 0xFFFFFFFFull)
         return context_fail(c, SWR_ERR_CAPACITY, "too many pixels for one swr_diff call");
-    uint8_t *pbuf = (uint8_t *)context_zeroed_scratch(c, 1, off_e + tiles * 256 * 4);
+    uint8_t *pbuf = (uint8_t *)context_zeroed_scratch(c, 1, off_e + tiles * 512 * 4);
     if (!pbuf)
         return context_last_code(c);
     d.qcnt = reinterpret_cast<uint32_t *>(pbuf + off_t) + tiles;
