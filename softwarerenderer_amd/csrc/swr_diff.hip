@@ -177,12 +177,8 @@ __device__ inline H3 pixel_ray(const DiffArgs &d, int px, int py)
     return {X, Y, 1.0};
 }
 
-// Window position of a clip-space vertex (w > 0): fp32 for decisions, fp64 for values.
-__device__ inline float2 to_win_f(const DiffArgs &d, int view, int v)
-{
-    const float4 h = d.clip[crow(d, view, v)];
-    return make_float2(d.sx * (h.x / h.w) + d.sx, -d.sy * (h.y / h.w) + d.sy);
-}
+// Window position of a clip-space vertex (w > 0): fp32 for decisions (tri_win), fp64 for
+// values.
 
 __device__ inline double2 to_win_d(const DiffArgs &d, const H3 &h)
 {
@@ -198,11 +194,6 @@ __device__ inline float edge_fn(float2 j, float2 k, float2 p)
 __device__ inline double edge_d(double2 j, double2 k, double2 p)
 {
     return (k.x - j.x) * (p.y - j.y) - (k.y - j.y) * (p.x - j.x);
-}
-
-__device__ inline bool w_positive(const DiffArgs &d, int view, int v)
-{
-    return d.clip[crow(d, view, v)].w > 0.0f;
 }
 
 // One neighbour pair as the antialiasing pass sees it.
@@ -255,13 +246,16 @@ __device__ inline PairVal pair_val(const DiffArgs &d, int view, const Pair &pr, 
 __device__ inline bool tri_win(const DiffArgs &d, int view, int t, float2 *v, int *vid)
 {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < 3; ++i)
         vid[i] = d.tris[3 * t + i];
-        if (!w_positive(d, view, vid[i]))
-            return false;
-        v[i] = to_win_f(d, view, vid[i]);
+    bool front = true;  // the three vertices' loads leave together
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float4 h = d.clip[crow(d, view, vid[i])];
+        front = front && h.w > 0.0f;
+        v[i] = make_float2(d.sx * (h.x / h.w) + d.sx, -d.sy * (h.y / h.w) + d.sy);
     }
-    return true;
+    return front;
 }
 
 constexpr int MARCH_STEPS = 8;
@@ -336,6 +330,11 @@ __device__ inline Pair eval_pair(const DiffArgs &d, int view, int px, int py, in
     if (!(area != 0.0f))
         return r;
     int from = -1;
+    int ad[3];  // the triangle's neighbours, loaded beside its vertex numbers: a step then waits
+                // for one load of these and one of the vertices
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        ad[e] = d.adj[3 * cur + e];
     for (int step = 0; step < MARCH_STEPS; ++step) {
         const float s = area > 0.0f ? 1.0f : -1.0f;
         float best = 2.0f;
@@ -356,18 +355,26 @@ __device__ inline Pair eval_pair(const DiffArgs &d, int view, int px, int py, in
         }
         if (be < 0)
             return r;  // the segment ends inside this triangle
-        const int n = d.adj[3 * cur + be];
+        const int n = be == 0 ? ad[0] : (be == 1 ? ad[1] : ad[2]);
         float2 nv[3];
-        int nvid[3];
+        int nvid[3], nad[3] = {-1, -1, -1};
         float an = 0.0f;
         bool interior = false;
+        if (n >= 0 && n < d.T) {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                nad[e] = d.adj[3 * n + e];
+        }
         if (n >= 0 && n < d.T && tri_win(d, view, n, nv, nvid)) {
             an = edge_fn(nv[0], nv[1], nv[2]);
             interior = an != 0.0f && ((an > 0.0f) == (area > 0.0f));
         }
         if (!interior) {
-            const int j = (be + 1) % 3, k = (be + 2) % 3;
-            if (v[k].x == v[j].x && v[k].y == v[j].y)
+            // vertices j = be + 1 and k = be + 2 of the triangle, by selects (a runtime index
+            // would put the arrays in memory)
+            const float2 vj = be == 0 ? v[1] : (be == 1 ? v[2] : v[0]);
+            const float2 vk = be == 0 ? v[2] : (be == 1 ? v[0] : v[1]);
+            if (vk.x == vj.x && vk.y == vj.y)
                 return r;  // a degenerate edge has no direction
             r.active = true;
             r.horiz = horiz;
@@ -375,8 +382,8 @@ __device__ inline Pair eval_pair(const DiffArgs &d, int view, int px, int py, in
             r.s = s;
             r.tri = cur;
             r.edge = be;
-            r.vj = vid[j];
-            r.vk = vid[k];
+            r.vj = be == 0 ? vid[1] : (be == 1 ? vid[2] : vid[0]);
+            r.vk = be == 0 ? vid[2] : (be == 1 ? vid[0] : vid[1]);
             r.front_is_p = pf;
             r.p_blended = (best < 0.5f) == pf;
             return r;
@@ -384,7 +391,7 @@ __device__ inline Pair eval_pair(const DiffArgs &d, int view, int px, int py, in
         int fe = -1;
 #pragma unroll
         for (int e = 0; e < 3; ++e)
-            if (d.adj[3 * n + e] == cur)
+            if (nad[e] == cur)
                 fe = e;
         if (fe < 0)
             return r;
@@ -395,6 +402,7 @@ __device__ inline Pair eval_pair(const DiffArgs &d, int view, int px, int py, in
         for (int i = 0; i < 3; ++i) {
             v[i] = nv[i];
             vid[i] = nvid[i];
+            ad[i] = nad[i];
         }
     }
     return r;
@@ -509,10 +517,12 @@ constexpr int ACC_PROBES = 32;   // one 16x16 tile: a few dozen vertices, the ta
 constexpr int ACC_VALS = 8;      // at most: clip x, y, w, attributes 0..4
 // values per slot with C attribute channels: clip x, y, w and the C attributes
 template <int C> constexpr int acc_vals() { return 3 + C; }
+// words of a slot: odd, so that the slots' values spread over the LDS banks
+template <int C> constexpr int acc_stride() { return acc_vals<C>() * 4 + 1; }
 // Each value is kept in four copies, picked by the pixel's (x, y) parity: the pixels of one
 // triangle are neighbours, and four copies cut the lanes of a wave that add into the same
 // LDS word (which serialise) about four times.  The flush sums the copies.
-constexpr int ACC_COPIES = 4;
+constexpr int ACC_COPIES = 4;  // (acc_stride counts on it)
 
 __device__ inline int acc_copy() { return (int)((threadIdx.x & 1u) | ((threadIdx.x >> 3) & 2u)); }
 
@@ -545,7 +555,7 @@ __device__ inline void acc_clip(const DiffArgs &d, const VertexAcc &A, int view,
 {
     const int sl = acc_slot(A, v);
     if (sl >= 0) {
-        float *x = &A.val[sl * acc_vals<C>() * ACC_COPIES + acc_copy()];
+        float *x = &A.val[sl * acc_stride<C>() + acc_copy()];
         atomicAdd(x + 0 * ACC_COPIES, gx);
         atomicAdd(x + 1 * ACC_COPIES, gy);
         atomicAdd(x + 2 * ACC_COPIES, gw);
@@ -564,7 +574,7 @@ __device__ inline void acc_vertex(const DiffArgs &d, const VertexAcc &A, int vie
 {
     const int sl = acc_slot(A, v);
     if (sl >= 0) {
-        float *x = &A.val[sl * acc_vals<C>() * ACC_COPIES + acc_copy()];
+        float *x = &A.val[sl * acc_stride<C>() + acc_copy()];
         atomicAdd(x + 0 * ACC_COPIES, gx);
         atomicAdd(x + 1 * ACC_COPIES, gy);
         atomicAdd(x + 2 * ACC_COPIES, gw);
@@ -579,31 +589,6 @@ __device__ inline void acc_vertex(const DiffArgs &d, const VertexAcc &A, int vie
 #pragma unroll
         for (int c = 0; c < C; ++c)
             atomicAdd(d.gattr + crow(d, view, v) * C + c, ga[c]);
-    }
-}
-
-// The same with the three slots already found (acc_slot; -1: straight to global memory).
-template <int C>
-__device__ inline void acc_triangle_at(const DiffArgs &d, const VertexAcc &A, int view,
-                                       const int (&v)[3], const int (&sl)[3],
-                                       const float (&g)[3][3 + C])
-{
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        if (sl[m] >= 0) {
-            float *x = &A.val[sl[m] * acc_vals<C>() * ACC_COPIES + acc_copy()];
-#pragma unroll
-            for (int k = 0; k < 3 + C; ++k)
-                atomicAdd(x + k * ACC_COPIES, g[m][k]);
-        } else {
-            float *gc = d.gclip + crow(d, view, v[m]) * 4;
-            atomicAdd(gc + 0, g[m][0]);
-            atomicAdd(gc + 1, g[m][1]);
-            atomicAdd(gc + 3, g[m][2]);
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-                atomicAdd(d.gattr + crow(d, view, v[m]) * C + c, g[m][3 + c]);
-        }
     }
 }
 
@@ -624,15 +609,6 @@ __device__ inline void acc_find3(const VertexAcc &A, const int (&v)[3], int (&sl
 }
 
 template <int C>
-__device__ inline void acc_triangle(const DiffArgs &d, const VertexAcc &A, int view,
-                                   const int (&v)[3], const float (&g)[3][3 + C])
-{
-    int sl[3];
-    acc_find3(A, v, sl);
-    acc_triangle_at<C>(d, A, view, v, sl, g);
-}
-
-template <int C>
 __device__ inline void acc_flush(const DiffArgs &d, const VertexAcc &A, int view)
 {
     for (int sl = threadIdx.x; sl < ACC_SLOTS; sl += blockDim.x) {
@@ -642,8 +618,8 @@ __device__ inline void acc_flush(const DiffArgs &d, const VertexAcc &A, int view
         float x[ACC_VALS];
 #pragma unroll
         for (int k = 0; k < acc_vals<C>(); ++k) {
-            const float4 q = *reinterpret_cast<const float4 *>(&A.val[(sl * acc_vals<C>() + k) * ACC_COPIES]);
-            x[k] = (q.x + q.y) + (q.z + q.w);
+            const float *q = &A.val[sl * acc_stride<C>() + k * ACC_COPIES];
+            x[k] = (q[0] + q[1]) + (q[2] + q[3]);
         }
         float *g = d.gclip + crow(d, view, v) * 4;
         if (x[0] != 0.0f) atomicAdd(g + 0, x[0]);
@@ -864,8 +840,6 @@ __device__ inline Pair unpack_pair(const PairLds &x, bool swap, bool horiz)
 // A workgroup's share of per-tile segments: TILES consecutive tiles, their lengths scanned
 // into s_off (s_off[k] = entries before tile k, s_off[TILES] = all), so the workgroup's threads
 // take the entries densely, one each.
-constexpr int TILES_PER_GROUP = 64;
-
 template <int TILES>
 __device__ inline void group_segments(const uint32_t *cnt, uint32_t tiles, uint32_t t0,
                                       uint32_t *s_off)
@@ -905,19 +879,21 @@ __device__ inline uint32_t group_tile(const uint32_t *s_off, uint32_t j)
 
 // The queued pairs, one lane each: the silhouette walk, the stored decision, and the tile
 // flags of active pairs.  A walk is a chain of dependent loads (adjacency, then the next
-// triangle's vertices), so the kernel is latency-bound: 1024 lanes per group of 64 tiles
-// take a group's queue in one pass where 256 lanes needed several in turn.
-constexpr int MARCH_THREADS = 1024;
+// triangle's vertices), so the kernel is latency-bound and wants every queued pair in flight
+// at once: a silhouette fills a tile's queue, so 256 lanes take 8 tiles.  64 views of 512x512:
+// 183 us with 1024 lanes per 64 tiles (a compute unit holds one such workgroup), 351 us with
+// 64 lanes per 8 tiles (several passes), 109 us now; one 256x256 view 30 -> 17 us.
+constexpr int MARCH_TILES = 8, MARCH_THREADS = 256;
 
 __global__ void __launch_bounds__(MARCH_THREADS) k_diff_march(DiffArgs d)
 {
-    __shared__ uint32_t s_off[TILES_PER_GROUP + 1];
-    const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * TILES_PER_GROUP;
-    group_segments<TILES_PER_GROUP>(d.qcnt, tiles, t0, s_off);
-    const uint32_t n = s_off[TILES_PER_GROUP];
+    __shared__ uint32_t s_off[MARCH_TILES + 1];
+    const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * MARCH_TILES;
+    group_segments<MARCH_TILES>(d.qcnt, tiles, t0, s_off);
+    const uint32_t n = s_off[MARCH_TILES];
     const size_t HW = (size_t)d.W * d.H;
     for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) {
-        const uint32_t t = group_tile<TILES_PER_GROUP>(s_off, j);
+        const uint32_t t = group_tile<MARCH_TILES>(s_off, j);
         const uint32_t k = d.queue[(size_t)(t0 + t) * 512 + (j - s_off[t])];
         const size_t i = k >> 1;
         const int dir = (int)(k & 1u);
@@ -1184,11 +1160,11 @@ template <int C>
 __global__ void __launch_bounds__(256) k_diff_backward(DiffArgs d)
 {
     __shared__ int s_key[ACC_SLOTS];
-    __shared__ __align__(16) float s_val[ACC_SLOTS * acc_vals<C>() * ACC_COPIES];
+    __shared__ __align__(16) float s_val[ACC_SLOTS * acc_stride<C>()];
     __shared__ PairLds s_h[TP_H], s_v[TP_V];
     for (int sl = threadIdx.x; sl < ACC_SLOTS; sl += blockDim.x)
         s_key[sl] = -1;
-    for (int k = threadIdx.x; k < ACC_SLOTS * acc_vals<C>() * ACC_COPIES / 4; k += blockDim.x)
+    for (int k = threadIdx.x; k < ACC_SLOTS * acc_stride<C>() / 4; k += blockDim.x)
         reinterpret_cast<float4 *>(s_val)[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     PixelIdx pi;
     const bool valid = pixel_of_thread(d, pi);
@@ -1221,22 +1197,39 @@ __device__ inline int row_prev(int v, int edge)
 }
 
 // Every pixel's interpolation under dL/dimage.  Neighbouring pixels mostly show the same
-// triangle (82% of horizontal pairs on the 41k-vertex sphere), so before the LDS adds the
-// lanes of a pixel row merge their 18 gradient values pairwise, then in fours and eights
-// (a lane keeps its values when its partner shows another triangle): about half the LDS
-// atomics, which serialise on the shared vertices, go away.
+// triangle (82% of horizontal pairs on the 41k-vertex sphere), so the lanes of a pixel row
+// first merge their gradient values pairwise, then in fours and eights (a lane keeps its values
+// when its partner shows another triangle).  The sums per vertex of the tile then go through
+// lists, not through LDS float atomics, which take about two cycles per lane whatever the
+// banks: a lane stores its merged values (3 corners of NV) with plain LDS writes, links each
+// corner into its vertex's list with one exchange (3 atomics instead of 3 NV), and after a
+// barrier a thread per (vertex, value) walks the vertex's two lists (of even and odd waves, so
+// that the chains of reads overlap), adds in fp64 and flushes: neighbouring lanes add to
+// neighbouring words of a gradient row, a third of the memory requests of a lane per vertex.
+// Tiles of background alone leave at once.  64 views of 512x512 (41k vertices): 485 us with LDS
+// float atomics and a flush of one lane per vertex, 427 us with lists and that flush, 252 us
+// now (136 us without any accumulation); 16 terrain views of 768x768: 494 -> 346 us.
+constexpr uint32_t LIST_END = 0xFFFFu;
+
 template <int C>
 __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
 {
     constexpr int NV = 3 + C;
     __shared__ int s_key[ACC_SLOTS];
-    __shared__ __align__(16) float s_val[ACC_SLOTS * acc_vals<C>() * ACC_COPIES];
-    for (int sl = threadIdx.x; sl < ACC_SLOTS; sl += blockDim.x)
-        s_key[sl] = -1;
-    for (int k = threadIdx.x; k < ACC_SLOTS * acc_vals<C>() * ACC_COPIES / 4; k += blockDim.x)
-        reinterpret_cast<float4 *>(s_val)[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    __shared__ uint32_t s_head[2][ACC_SLOTS];
+    __shared__ uint16_t s_next[3 * 256];
+    constexpr int ST = NV | 1;               // odd: lanes' entries spread over the banks
+    __shared__ float s_val[3 * 256 * ST];    // entry m * 256 + thread: corner m of a lane
+    __shared__ uint8_t s_used[ACC_SLOTS];    // the occupied slots, packed
+    __shared__ uint32_t s_cnt[4];
     PixelIdx pi;
     const bool valid = pixel_of_thread(d, pi);
+    const int t0 = valid ? id_tri(d, pi.view, d.ids[pi.i]) : -1;
+    if (!__syncthreads_or(t0 >= 0))
+        return;  // background: nothing to add
+    static_assert(ACC_SLOTS == 256, "a slot per thread");
+    s_key[threadIdx.x] = -1;
+    s_head[0][threadIdx.x] = s_head[1][threadIdx.x] = LIST_END;
     int tri = -1, vid[3] = {0, 0, 0};
     float g[3][NV];
 #pragma unroll
@@ -1244,17 +1237,15 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
 #pragma unroll
         for (int k = 0; k < NV; ++k)
             g[m][k] = 0.0f;
-    if (valid) {
-        const uint32_t id = d.ids[pi.i];
+    if (t0 >= 0) {
         Bary B;
-        const int t = id_tri(d, pi.view, id);
-        if (t >= 0 && bary_at(d, pi.view, t, pi.px, pi.py, B)) {
+        if (bary_at(d, pi.view, t0, pi.px, pi.py, B)) {
             double gc[C];
 #pragma unroll
             for (int c = 0; c < C; ++c)
                 gc[c] = grad_image(d, pi.i, C, c);
             bary_grads<C>(d, B, gc, g);
-            tri = t;
+            tri = t0;
 #pragma unroll
             for (int m = 0; m < 3; ++m)
                 vid[m] = B.v[m];
@@ -1278,16 +1269,69 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
         }                                                                                      \
         keep = keep && !give;                                                                  \
     }
-    SWR_MERGE(1)
-    SWR_MERGE(2)
-    SWR_MERGE(4)
+    if (__ballot(keep) != 0ull) {
+        SWR_MERGE(1)
+        SWR_MERGE(2)
+        SWR_MERGE(4)
+    }
 #undef SWR_MERGE
     __syncthreads();
-    const VertexAcc A{s_key, s_val};
-    if (keep)
-        acc_triangle<C>(d, A, pi.view, vid, g);
+    const VertexAcc A{s_key, nullptr};
+    if (keep) {
+        int sl[3];
+        acc_find3(A, vid, sl);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const uint32_t e = (uint32_t)m * 256u + threadIdx.x;
+            if (sl[m] >= 0) {
+#pragma unroll
+                for (int k = 0; k < NV; ++k)
+                    s_val[e * ST + k] = g[m][k];
+                s_next[e] = (uint16_t)atomicExch(&s_head[(threadIdx.x >> 6) & 1u][sl[m]], e);
+            } else {  // no slot for this vertex
+                float *gc = d.gclip + crow(d, pi.view, vid[m]) * 4;
+                atomicAdd(gc + 0, g[m][0]);
+                atomicAdd(gc + 1, g[m][1]);
+                atomicAdd(gc + 3, g[m][2]);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    atomicAdd(d.gattr + crow(d, pi.view, vid[m]) * C + c, g[m][3 + c]);
+            }
+        }
+    }
     __syncthreads();
-    acc_flush<C>(d, A, pi.view);
+    const bool used = s_key[threadIdx.x] >= 0;
+    const unsigned long long mu = __ballot(used);
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    if (lane == 0)
+        s_cnt[w] = (uint32_t)__popcll(mu);
+    __syncthreads();
+    uint32_t before = 0, n = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+        before += q < w ? s_cnt[q] : 0u;
+        n += s_cnt[q];
+    }
+    if (used)
+        s_used[before + (uint32_t)__popcll(mu & ((1ull << lane) - 1ull))] = (uint8_t)threadIdx.x;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n * NV; i += 256) {
+        const uint32_t sl = s_used[i / NV], k = i % NV;
+        uint32_t e0 = s_head[0][sl], e1 = s_head[1][sl];
+        double x = 0.0;
+        while (e0 != LIST_END || e1 != LIST_END) {
+            const bool h0 = e0 != LIST_END, h1 = e1 != LIST_END;
+            const uint32_t a0 = h0 ? e0 : 0u, a1 = h1 ? e1 : 0u;
+            const float v0 = s_val[a0 * ST + k], v1 = s_val[a1 * ST + k];
+            e0 = h0 ? s_next[a0] : LIST_END;
+            e1 = h1 ? s_next[a1] : LIST_END;
+            x += (double)(h0 ? v0 : 0.0f) + (double)(h1 ? v1 : 0.0f);
+        }
+        const size_t row = crow(d, pi.view, s_key[sl]);
+        float *to = k < 3 ? d.gclip + row * 4 + (k == 2 ? 3 : k) : d.gattr + row * C + (k - 3);
+        if (x != 0.0)
+            atomicAdd(to, (float)x);
+    }
 }
 
 // ---- what the antialiasing adds to the gradients ---------------------------------------------
@@ -1550,10 +1594,10 @@ static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const
     const uint32_t blocks = (uint32_t)((size_t)d.tiles_per_view * d.V);
     if (!blocks)
         return hipSuccess;
-    const uint32_t groups = (blocks + TILES_PER_GROUP - 1) / TILES_PER_GROUP;
     if (which == 0) {
         hipLaunchKernelGGL(k_diff_interp<C>, dim3(blocks), dim3(256), 0, s, d);
-        hipLaunchKernelGGL(k_diff_march, dim3(groups), dim3(MARCH_THREADS), 0, s, d);
+        hipLaunchKernelGGL(k_diff_march, dim3((blocks + MARCH_TILES - 1) / MARCH_TILES),
+                           dim3(MARCH_THREADS), 0, s, d);
         hipLaunchKernelGGL(k_diff_blend<C>, dim3(blocks), dim3(256), 0, s, d);
     } else {
         if (d.pairs == 2) {
