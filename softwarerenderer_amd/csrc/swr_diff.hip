@@ -80,10 +80,12 @@ struct DiffArgs {
                        // bit 1 some pair to the right of its last column, bit 2 some pair
                        // below its last row
     // per (view, tile) b: the pairs that need the silhouette walk (pair index 2 * pixel +
-    // dir) at queue[b * 512 ..) with qcnt[b] entries, and the active ones of the tile's own
-    // pairs (the blend pass lists them) at elist[b * 512 ..) with ecnt[b] entries
+    // dir) at queue[b * 512 ..) with qcnt[b] entries; and per region of `region_tiles`
+    // consecutive tiles r: its active pairs (the blend pass appends them) at
+    // elist[r * region_tiles * 512 ..) with ecnt[r] entries
     uint32_t *queue, *qcnt;
     uint32_t *elist, *ecnt;
+    uint32_t region_tiles;
     int row_keys;  // 1: clip rows fit the int keys of the edge backward's table
     int pairs;     // 0: evaluate, 1: evaluate and store, 2: load the stored decisions
     // several meshes (null for one): per view, the clip row of global vertex g is
@@ -195,6 +197,10 @@ __device__ inline double edge_d(double2 j, double2 k, double2 p)
 {
     return (k.x - j.x) * (p.y - j.y) - (k.y - j.y) * (p.x - j.x);
 }
+
+// The active pairs' lists: one per EDGE_REGIONS-th of the tiles (a counter each: one for all
+// tiles would serialise their atomics).
+constexpr uint32_t EDGE_REGIONS = 256;
 
 // One neighbour pair as the antialiasing pass sees it.
 struct Pair {
@@ -736,7 +742,8 @@ __device__ inline void interp_pixel(const DiffArgs &d, const PixelIdx &pi, bool 
     }
     if (threadIdx.x == 0) {
         d.tflag[pi.tile] = 0u;
-        d.ecnt[pi.tile] = 0u;  // the blend pass fills it for tiles with an active pair
+        if (pi.tile < (int)EDGE_REGIONS)
+            d.ecnt[pi.tile] = 0u;  // the blend pass adds to it
     }
     // this pixel's two pairs (to the right, below): decided here unless a silhouette walk
     // is needed
@@ -1021,7 +1028,28 @@ __global__ void __launch_bounds__(256) k_diff_blend(DiffArgs d)
     const bool right = valid && (tile_own(s_h, s_v, 0).flags & 1),
                down = valid && (tile_own(s_h, s_v, 1).flags & 1);
     const uint32_t k0 = right || down ? (uint32_t)(2 * pi.i) : 0u;
-    tile_append2(d.elist + (size_t)b * 512, d.ecnt + b, right, k0, down, k0 + 1u);
+    // one global append per tile, spread over EDGE_REGIONS counters
+    __shared__ uint32_t s_n, s_base;
+    const unsigned long long mr = __ballot(right), md = __ballot(down);
+    const uint32_t lane = threadIdx.x & 63u, nw = (uint32_t)(__popcll(mr) + __popcll(md));
+    if (threadIdx.x == 0)
+        s_n = 0u;
+    __syncthreads();
+    uint32_t at = 0;
+    if (lane == 0 && nw)
+        at = atomicAdd(&s_n, nw);
+    at = __shfl(at, 0, 64);
+    __syncthreads();
+    const uint32_t region = (uint32_t)b / d.region_tiles;
+    if (threadIdx.x == 0 && s_n)
+        s_base = atomicAdd(d.ecnt + region, s_n);
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint32_t *to = d.elist + (size_t)region * d.region_tiles * 512 + s_base + at;
+    if (right)
+        to[__popcll(mr & below)] = k0;
+    if (down)
+        to[__popcll(mr) + __popcll(md & below)] = k0 + 1u;
     if (!valid)
         return;
     const size_t i = pi.i;
@@ -1340,48 +1368,58 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
 // pixel's half, B is the front pixel and the source the other pixel's colour, else B is the
 // other pixel and the source the silhouette triangle's colour at the crossing.  Either way the
 // source is a triangle's interpolation along a ray, so all lanes run the same code: B's and
-// the source's interpolation, forward and backward, and the crossing's derivatives, whose
-// gradients join those of the triangle that owns the edge.  Bound by the latency of that chain
-// (dependent loads, fp64 divisions), so it is kept short: with a lane per pixel and its four
-// pairs in turn, three divergent cases each, one 256x256 view took 79 us and 64 views of
-// 512x512 553 us (beside the interior kernel); now 30 and 171 us.
+// the source's interpolation, forward and backward, and the crossing's derivatives.  Bound by the latency of that chain
+// (dependent loads, fp64 divisions), so it is kept short and every wave gets 64 pairs: pairs
+// cluster on silhouettes, and a wave per 16 tiles left most waves idle behind a few long ones.
+// One 256x256 view / 64 views of 512x512 / 16 terrain views of 768x768, beside the interior
+// kernel: 79 / 553 / 1007 us with a lane per pixel and its four pairs in turn, 31 / 67 / 347 us
+// with a lane per pair and a wave per 16 tiles, 20 / 56 / 146 us now.
 //
-// Gradients are summed in an LDS table keyed by clip row (neighbouring silhouette pairs share
-// vertices), one wave per table; a row that finds no slot goes to global memory.
-constexpr int EDGE_TILES = 16;   // tiles per workgroup of one wave
-constexpr int EDGE_SLOTS = 128;  // power of two
+// Neighbouring silhouette pairs share vertices: a wave takes 64 pairs at a time, a pair stores
+// its 8 entries (two triangles' corners, the window gradients of the edge's ends), each rounded
+// to fp32 by itself, with plain LDS writes and links each into its clip row's list; a lane per
+// (row, value) then adds the list in fp64 and flushes, as in the interior kernel (LDS float
+// atomics took 309 us instead of 242 us on the terrain, alone and before the even split).  A
+// row that finds no slot goes to global memory.
+constexpr int EDGE_SLOTS = 256;  // power of two
 constexpr int EDGE_PROBES = 8;
-constexpr int EDGE_COPIES = 2;   // of each value, picked by lane parity
+constexpr int EDGE_ENTRIES = 8;  // per pair
 
 template <int C>
-struct EdgeAcc {
-    static constexpr int STRIDE = (3 + C) * EDGE_COPIES + 1;  // odd: slots spread over the banks
+struct EdgeLists {
+    static constexpr int NV = 3 + C, ST = NV | 1;  // odd: entries spread over the banks
     int key[EDGE_SLOTS];
-    float val[EDGE_SLOTS * STRIDE];
+    uint32_t head[EDGE_SLOTS];
+    uint16_t next[EDGE_ENTRIES * 64];
+    uint8_t used[EDGE_SLOTS];
+    float val[EDGE_ENTRIES * 64 * ST];
 };
 
-// Adds {clip x, y, w, attributes} to row `row`; attr = false: the clip part only.
+// Entry `n` of this lane's pair: {clip x, y, w, attributes} of clip row `row`.
 template <int C>
-__device__ inline void edge_add(const DiffArgs &d, EdgeAcc<C> &A, size_t row,
-                                const float (&g)[3 + C], bool attr)
+__device__ inline void edge_add(const DiffArgs &d, EdgeLists<C> &A, int n, size_t row,
+                                const float (&g)[3 + C])
 {
+    constexpr int NV = 3 + C;
     int slot = -1;
     if (d.row_keys) {
-        const unsigned h = ((unsigned)row * 2654435761u) >> 25;  // 7 bits: EDGE_SLOTS
+        const unsigned h = ((unsigned)row * 2654435761u) >> 24;  // 8 bits: EDGE_SLOTS
 #pragma unroll 1
         for (int probe = 0; probe < EDGE_PROBES && slot < 0; ++probe) {
             const int sl = (int)((h + (unsigned)probe) & (EDGE_SLOTS - 1));
-            const int old = atomicCAS(&A.key[sl], -1, (int)row);
+            int old = __atomic_load_n(&A.key[sl], __ATOMIC_RELAXED);
+            if (old == -1)
+                old = atomicCAS(&A.key[sl], -1, (int)row);
             if (old == -1 || old == (int)row)
                 slot = sl;
         }
     }
     if (slot >= 0) {
-        float *x = &A.val[slot * EdgeAcc<C>::STRIDE + (int)(threadIdx.x & (EDGE_COPIES - 1))];
+        const uint32_t e = (uint32_t)n * 64u + threadIdx.x;
 #pragma unroll
-        for (int k = 0; k < 3 + C; ++k)
-            if (k < 3 || attr)
-                atomicAdd(x + k * EDGE_COPIES, g[k]);
+        for (int k = 0; k < NV; ++k)
+            A.val[e * EdgeLists<C>::ST + k] = g[k];
+        A.next[e] = (uint16_t)atomicExch(&A.head[slot], e);
         return;
     }
     atomicAdd(d.gclip + row * 4 + 0, g[0]);
@@ -1389,27 +1427,35 @@ __device__ inline void edge_add(const DiffArgs &d, EdgeAcc<C> &A, size_t row,
     atomicAdd(d.gclip + row * 4 + 3, g[2]);
 #pragma unroll
     for (int c = 0; c < C; ++c)
-        if (attr)
-            atomicAdd(d.gattr + row * C + c, g[3 + c]);
+        atomicAdd(d.gattr + row * C + c, g[3 + c]);
 }
 
+// Adds every list to the gradients: a lane per (row, value), neighbouring lanes to
+// neighbouring words of a gradient row.
 template <int C>
-__device__ inline void edge_flush(const DiffArgs &d, const EdgeAcc<C> &A)
+__device__ inline void edge_flush(const DiffArgs &d, EdgeLists<C> &A)
 {
-    static_assert(EDGE_COPIES == 2, "the flush adds two copies");
-    for (int sl = threadIdx.x; sl < EDGE_SLOTS; sl += 64) {
-        const int row = A.key[sl];
-        if (row < 0)
-            continue;
-        const float *x = &A.val[sl * EdgeAcc<C>::STRIDE];
+    constexpr uint32_t NV = 3 + C;
+    const uint32_t lane = threadIdx.x;
+    uint32_t n = 0;
 #pragma unroll
-        for (int k = 0; k < 3 + C; ++k) {
-            const float v = x[k * EDGE_COPIES] + x[k * EDGE_COPIES + 1];
-            float *to = k < 3 ? d.gclip + (size_t)row * 4 + (k == 2 ? 3 : k)
-                              : d.gattr + (size_t)row * C + (k - 3);
-            if (v != 0.0f)
-                atomicAdd(to, v);
-        }
+    for (uint32_t q = 0; q < EDGE_SLOTS / 64; ++q) {
+        const bool used = A.key[q * 64 + lane] >= 0;
+        const unsigned long long m = __ballot(used);
+        if (used)
+            A.used[n + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)(q * 64 + lane);
+        n += (uint32_t)__popcll(m);
+    }
+    lds_sync();
+    for (uint32_t i = lane; i < n * NV; i += 64) {
+        const uint32_t sl = A.used[i / NV], k = i % NV;
+        double x = 0.0;
+        for (uint32_t e = A.head[sl]; e != LIST_END; e = A.next[e])
+            x += (double)A.val[e * EdgeLists<C>::ST + k];
+        const size_t row = (size_t)A.key[sl];
+        float *to = k < 3 ? d.gclip + row * 4 + (k == 2 ? 3 : k) : d.gattr + row * C + (k - 3);
+        if (x != 0.0)
+            atomicAdd(to, (float)x);
     }
 }
 
@@ -1424,7 +1470,7 @@ __device__ inline void window_grad(const DiffArgs &d, const H3 &h, double gx, do
 }
 
 template <int C>
-__device__ inline void backward_pair(const DiffArgs &d, EdgeAcc<C> &A, uint32_t k)
+__device__ inline void backward_pair(const DiffArgs &d, EdgeLists<C> &A, uint32_t k)
 {
     const size_t HW = (size_t)d.W * d.H;
     const size_t i = k >> 1;
@@ -1488,61 +1534,76 @@ __device__ inline void backward_pair(const DiffArgs &d, EdgeAcc<C> &A, uint32_t 
                 dldt * pv.tj.y + dlda * pv.aj.y, wj);
     window_grad(d, load_h(d, view, pr.vk), dldt * pv.tk.x + dlda * pv.ak.x,
                 dldt * pv.tk.y + dlda * pv.ak.y, wk);
-    // the triangle that owns the edge is the source's, or mostly the front pixel's own
-    const bool in_s = has_s && tri_s == pr.tri, in_b = !in_s && has_b && tri_b == pr.tri;
-    const auto triangle = [&](const Bary &T, const double *gc, bool own) {
+    const auto triangle = [&](const Bary &T, const double *gc, int n0) {
         float out[3][3 + C];
         bary_grads<C>(d, T, gc, out);
 #pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            if (own) {
-#pragma unroll
-                for (int n = 0; n < 3; ++n)
-                    out[m][n] += T.v[m] == pr.vj ? wj[n] : (T.v[m] == pr.vk ? wk[n] : 0.0f);
-            }
-            edge_add<C>(d, A, crow(d, view, T.v[m]), out[m], true);
-        }
+        for (int m = 0; m < 3; ++m)
+            edge_add<C>(d, A, n0 + m, crow(d, view, T.v[m]), out[m]);
     };
     if (has_s)
-        triangle(S, gs, in_s);
+        triangle(S, gs, 0);
     if (has_b)
-        triangle(B, gb, in_b);
-    if (!in_s && !in_b) {
-        float out[3 + C];
+        triangle(B, gb, 3);
+    // two entries without attributes
+    float out[3 + C];
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-            out[3 + c] = 0.0f;
+    for (int c = 0; c < C; ++c)
+        out[3 + c] = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
+    for (int v = 0; v < 2; ++v) {
 #pragma unroll
-            for (int n = 0; n < 3; ++n)
-                out[n] = v == 0 ? wj[n] : wk[n];
-            edge_add<C>(d, A, crow(d, view, v == 0 ? pr.vj : pr.vk), out, false);
-        }
+        for (int n = 0; n < 3; ++n)
+            out[n] = v == 0 ? wj[n] : wk[n];
+        edge_add<C>(d, A, 6 + v, crow(d, view, v == 0 ? pr.vj : pr.vk), out);
     }
 }
 
 template <int C>
-__global__ void __launch_bounds__(64) k_diff_bwd_edges(DiffArgs d)
+__global__ void __launch_bounds__(64) k_diff_bwd_edges(DiffArgs d, uint32_t regions)
 {
-    __shared__ EdgeAcc<C> A;
-    __shared__ uint32_t s_off[EDGE_TILES + 1];
-    const uint32_t tiles = (uint32_t)(d.tiles_per_view * d.V), t0 = blockIdx.x * EDGE_TILES;
-    group_segments<EDGE_TILES>(d.ecnt, tiles, t0, s_off);
-    const uint32_t n = s_off[EDGE_TILES];
-    if (n == 0)
-        return;
-    for (int sl = threadIdx.x; sl < EDGE_SLOTS; sl += 64)
-        A.key[sl] = -1;
-    for (int k = threadIdx.x; k < EDGE_SLOTS * EdgeAcc<C>::STRIDE; k += 64)
-        A.val[k] = 0.0f;
-    __syncthreads();
-    for (uint32_t j = threadIdx.x; j < n; j += 64) {
-        const uint32_t t = group_tile<EDGE_TILES>(s_off, j);
-        backward_pair<C>(d, A, d.elist[(size_t)(t0 + t) * 512 + (j - s_off[t])]);
+    __shared__ EdgeLists<C> A;
+    __shared__ uint32_t s_off[EDGE_REGIONS + 1];  // pairs before region r
+    const uint32_t lane = threadIdx.x;
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < EDGE_REGIONS / 64; ++q) {
+        const uint32_t r = q * 64 + lane;
+        uint32_t c = r < regions ? d.ecnt[r] : 0u, v = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = __shfl_up(v, o, 64);
+            v += (int)lane >= o ? u : 0u;
+        }
+        s_off[r] = n + v - c;
+        n += __shfl(v, 63, 64);
     }
-    __syncthreads();
-    edge_flush<C>(d, A);
+    if (lane == 0)
+        s_off[EDGE_REGIONS] = n;
+    lds_sync();
+    for (uint32_t j0 = blockIdx.x * 64; j0 < n; j0 += gridDim.x * 64) {
+#pragma unroll
+        for (int q = 0; q < EDGE_SLOTS / 64; ++q) {
+            A.key[q * 64 + lane] = -1;
+            A.head[q * 64 + lane] = LIST_END;
+        }
+        lds_sync();
+        const uint32_t j = j0 + lane;
+        if (j < n) {
+            uint32_t lo = 0, hi = EDGE_REGIONS;  // the last region with s_off <= j
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (s_off[mid] <= j)
+                    lo = mid;
+                else
+                    hi = mid;
+            }
+            backward_pair<C>(d, A, d.elist[(size_t)lo * d.region_tiles * 512 + (j - s_off[lo])]);
+        }
+        lds_sync();
+        edge_flush<C>(d, A);
+        lds_sync();  // the lists are cleared for the next 64 pairs
+    }
 }
 
 // grad_attributes += sum over the views that see the vertex (in view order) of the
@@ -1588,6 +1649,8 @@ struct SideStream {
     hipEvent_t fork = nullptr, join = nullptr;
 };
 
+constexpr uint32_t EDGE_WAVES = 2048;
+
 template <int C>
 static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const SideStream &side)
 {
@@ -1611,8 +1674,10 @@ static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const
                     return e;
                 se = side.s;
             }
-            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3((blocks + EDGE_TILES - 1) / EDGE_TILES),
-                               dim3(64), 0, se, d);
+            // as many waves as the GPU holds (two per SIMD), or a wave per 64 possible pairs
+            const uint32_t waves = blocks < EDGE_WAVES / 8 ? blocks * 8 : EDGE_WAVES;
+            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3(waves), dim3(64), 0, se, d,
+                               (blocks + d.region_tiles - 1) / d.region_tiles);
             hipLaunchKernelGGL(k_diff_bwd_interior<C>, dim3(blocks), dim3(256), 0, s, d);
             if (fork) {
                 hipError_t e = hipEventRecord(side.join, side.s);
@@ -1741,14 +1806,16 @@ static int diff_run(swr_context *c, const swr_diff_desc *dd, const float *gimage
     // The forward stores its pair decisions; a backward over the same buffers and sizes
     // reuses them instead of walking the silhouettes again.
     // layout: flags [2 px] u8, data [2 px] int2, per tile: flags, queue and list lengths
-    // u32, queue [tiles][512] u32, list [tiles][512] u32
+    // u32, queue [tiles][512] u32, which the active pairs' lists take over: the blend pass
+    // writes them once the march pass has read the queue
     const size_t tiles = (size_t)d.tiles_per_view * d.V, off_f = 0,
                  off_d = (off_f + px * 2 + 15) & ~(size_t)15, off_t = off_d + px * 2 * sizeof(int2),
-                 off_q = (off_t + tiles * 12 + 15) & ~(size_t)15, off_e = off_q + tiles * 512 * 4;
+                 off_q = (off_t + tiles * 12 + 15) & ~(size_t)15;
+    d.region_tiles = (uint32_t)((tiles + EDGE_REGIONS - 1) / EDGE_REGIONS);
     d.row_keys = rows <= 0x7FFFFFFFull ? 1 : 0;
     if (px * 2 > 0xFFFFFFFFull)
         return context_fail(c, SWR_ERR_CAPACITY, "too many pixels for one swr_diff call");
-    uint8_t *pbuf = (uint8_t *)context_zeroed_scratch(c, 1, off_e + tiles * 512 * 4);
+    uint8_t *pbuf = (uint8_t *)context_zeroed_scratch(c, 1, off_q + tiles * 512 * 4);
     if (!pbuf)
         return context_last_code(c);
     d.qcnt = reinterpret_cast<uint32_t *>(pbuf + off_t) + tiles;
@@ -1757,7 +1824,7 @@ static int diff_run(swr_context *c, const swr_diff_desc *dd, const float *gimage
     d.pdata = reinterpret_cast<int2 *>(pbuf + off_d);
     d.tflag = reinterpret_cast<uint32_t *>(pbuf + off_t);
     d.queue = reinterpret_cast<uint32_t *>(pbuf + off_q);
-    d.elist = reinterpret_cast<uint32_t *>(pbuf + off_e);
+    d.elist = d.queue;
     const uint64_t tag[9] = {(uint64_t)(uintptr_t)q.clip,      (uint64_t)(uintptr_t)q.triangles,
                              (uint64_t)(uintptr_t)q.adjacency, (uint64_t)(uintptr_t)q.ids,
                              (uint64_t)(uintptr_t)q.depth,     (uint64_t)(uintptr_t)pbuf,
