@@ -67,7 +67,7 @@ struct swr_context {
 
     // arenas
     DevBuf idx, attr0, wverts, app, app_ex, live, grp, grp_ex, scan_tmp, prims, pk_a, pv_a, pk_b, pv_b,
-        ranges, hist, hist_ex, hist_tmp, status, tgt[3], log, logcount,
+        ranges, hist, status, tgt[3], log, logcount,
         bigq,       // per-primitive first pair index
         clipq,      // triangles queued for the clipper
         clipq_cnt,  // its per-region counters
@@ -417,7 +417,7 @@ struct Arenas {
     uint32_t *ranges = nullptr;
     float *prims = nullptr;
     uint32_t *bigq = nullptr, *pk_a = nullptr, *pv_a = nullptr, *pk_b = nullptr, *pv_b = nullptr;
-    uint32_t *hist = nullptr, *hist_ex = nullptr, *hist_tmp = nullptr;
+    uint32_t *hist = nullptr;
     uint32_t *chunk_kept = nullptr;
     uint64_t prim_cap = 0, pair_cap = 0;
     uint32_t G = 1;  // radix sort workgroups
@@ -447,7 +447,8 @@ uint32_t sort_blocks(uint64_t pair_cap)
     return (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, pair_cap / 4096));
 }
 
-size_t hist_bytes(uint32_t G) { return (size_t)256 * G * 4; }
+// the radix blocks' counts and the digits' totals
+size_t hist_bytes(uint32_t G) { return (size_t)256 * (G + 1) * 4; }
 // kept-pair counts of the expansion chunks (256 slots at the least)
 size_t chunk_kept_bytes(uint64_t pair_cap) { return (pair_cap / 256 + 1) * 4; }
 // the expansion chunk launch_expand uses for a tuning value
@@ -455,7 +456,6 @@ int expand_chunk_of(int tuned)
 {
     return (tuned == 256 || tuned == 512 || tuned == 2048 || tuned == 4096) ? tuned : 1024;
 }
-size_t hist_tmp_bytes(uint32_t G) { return scan_tmp_elems((uint64_t)256 * G) * 4; }
 
 // ---- the no-allocation draw's scratch ------------------------------------------------------
 // One array per GPU, in the code object's device memory: swr_draw_elements_noalloc carves all
@@ -534,7 +534,7 @@ bool carve_arenas(unsigned char *base, size_t bytes, size_t T, uint64_t ngrp, ui
     size_t rest = bytes - off - A.prim_cap * rec_bytes - slack;
     uint64_t pairs = rest / 16;
     A.G = sort_blocks(pairs);
-    const size_t hb = 2 * hist_bytes(A.G) + hist_tmp_bytes(A.G) + chunk_kept_bytes(pairs) + 256;
+    const size_t hb = hist_bytes(A.G) + chunk_kept_bytes(pairs) + 256;
     if (hb >= rest)
         return false;
     pairs = (rest - hb) / 16;
@@ -548,8 +548,6 @@ bool carve_arenas(unsigned char *base, size_t bytes, size_t T, uint64_t ngrp, ui
     A.pk_b = (uint32_t *)take(A.pair_cap * 4);
     A.pv_b = (uint32_t *)take(A.pair_cap * 4);
     A.hist = (uint32_t *)take(hist_bytes(A.G));
-    A.hist_ex = (uint32_t *)take(hist_bytes(A.G));
-    A.hist_tmp = (uint32_t *)take(hist_tmp_bytes(A.G));
     A.chunk_kept = (uint32_t *)take(chunk_kept_bytes(A.pair_cap));
     return off <= bytes;
 }
@@ -708,8 +706,6 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
             HIP_TRY(c, ensure(c, c->pv_b, c->pair_cap * 4));
             A.G = sort_blocks(c->pair_cap);
             HIP_TRY(c, ensure(c, c->hist, hist_bytes(A.G)));
-            HIP_TRY(c, ensure(c, c->hist_ex, hist_bytes(A.G)));
-            HIP_TRY(c, ensure(c, c->hist_tmp, hist_tmp_bytes(A.G)));
             HIP_TRY(c, ensure(c, c->chunk_kept, chunk_kept_bytes(c->pair_cap)));
             A.prims = (float *)c->prims.p;
             A.bigq = (uint32_t *)c->bigq.p;
@@ -718,8 +714,6 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
             A.pk_b = (uint32_t *)c->pk_b.p;
             A.pv_b = (uint32_t *)c->pv_b.p;
             A.hist = (uint32_t *)c->hist.p;
-            A.hist_ex = (uint32_t *)c->hist_ex.p;
-            A.hist_tmp = (uint32_t *)c->hist_tmp.p;
             A.chunk_kept = (uint32_t *)c->chunk_kept.p;
             A.prim_cap = c->prim_cap;
             A.pair_cap = c->pair_cap;
@@ -815,8 +809,7 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
         sb.keys_b = A.pk_b;
         sb.vals_b = A.pv_b;
         sb.hist = A.hist;
-        sb.hist_ex = A.hist_ex;
-        sb.scan_tmp = A.hist_tmp;
+        sb.tot = A.hist + (size_t)256 * G;
         sb.ranges = A.ranges;
         sb.blocks = G;
         sb.chunk_kept = A.chunk_kept;
@@ -1028,10 +1021,8 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
         HIP_TRY(c, ensure(c, c->pv_a, c->pair_cap * 4));
         HIP_TRY(c, ensure(c, c->pk_b, c->pair_cap * 4));
         HIP_TRY(c, ensure(c, c->pv_b, c->pair_cap * 4));
-        uint32_t G = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, c->pair_cap / 4096));
-        HIP_TRY(c, ensure(c, c->hist, (size_t)256 * G * 4));
-        HIP_TRY(c, ensure(c, c->hist_ex, (size_t)256 * G * 4));
-        HIP_TRY(c, ensure(c, c->hist_tmp, scan_tmp_elems((uint64_t)256 * G) * 4));
+        const uint32_t G = sort_blocks(c->pair_cap);
+        HIP_TRY(c, ensure(c, c->hist, hist_bytes(G)));
         A.frags = (float *)c->prims.p;
         A.keys = (uint32_t *)c->pk_a.p;
         A.vals = (uint32_t *)c->pv_a.p;
@@ -1043,8 +1034,7 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
         sb.keys_b = (uint32_t *)c->pk_b.p;
         sb.vals_b = (uint32_t *)c->pv_b.p;
         sb.hist = (uint32_t *)c->hist.p;
-        sb.hist_ex = (uint32_t *)c->hist_ex.p;
-        sb.scan_tmp = (uint32_t *)c->hist_tmp.p;
+        sb.tot = sb.hist + (size_t)256 * G;
         sb.ranges = (uint32_t *)c->ranges.p;
         sb.blocks = G;
         HIP_TRY(c, sort_pairs(sb, g.status, tiles, c->stream));
@@ -1247,7 +1237,7 @@ int swr_destroy(swr_context *c)
     DevBuf *bufs[] = {&c->idx, &c->attr0, &c->wverts, &c->app, &c->app_ex, &c->live, &c->grp,
                       &c->grp_ex,
                       &c->scan_tmp, &c->prims, &c->pk_a, &c->pv_a, &c->pk_b, &c->pv_b,
-                      &c->ranges, &c->hist, &c->hist_ex, &c->hist_tmp, &c->status, &c->tgt[0],
+                      &c->ranges, &c->hist, &c->status, &c->tgt[0],
                       &c->tgt[1], &c->tgt[2], &c->log, &c->logcount, &c->bigq, &c->clipq,
                       &c->clipq_cnt, &c->chunk_kept, &c->vwin, &c->vmask, &c->vmod_out,
                       &c->zscratch[0], &c->zscratch[1], &c->diff_table};

@@ -7,12 +7,13 @@ namespace swr {
 
 struct SortBuffers {
     uint32_t *keys_a, *vals_a, *keys_b, *vals_b;
-    uint32_t *hist, *hist_ex, *scan_tmp;
+    uint32_t *hist, *tot;  // [256 * blocks] and [256]
     uint32_t *ranges;
-    uint32_t blocks;
+    uint32_t blocks;       // at most 1024
     const uint32_t *chunk_kept = nullptr;  // pairs kept per expansion chunk (nullptr: one run)
     uint32_t chunk = 0;                    // slots per expansion chunk
-    uint32_t *sorted_keys, *sorted_vals;  // set by sort_pairs
+    uint32_t *sorted_keys, *sorted_vals;  // set by sort_pairs (the keys unless `ranged`)
+    bool ranged = false;                  // sort_pairs wrote the tiles' ranges itself
 };
 
 // geometry (swr_geometry.hip)
@@ -55,9 +56,7 @@ hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uin
                                const uint2 *grp, uint2 *grp_ex, uint64_t ng, void *tmp,
                                unsigned long long *status, uint64_t cap_prims,
                                uint64_t cap_pairs, hipStream_t s);
-int radix_passes(uint32_t tiles);
-hipError_t sort_pairs(SortBuffers &sb, const unsigned long long *status, uint32_t tiles,
-                      hipStream_t s);
+hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tiles, hipStream_t s);
 hipError_t launch_ranges(const SortBuffers &sb, const unsigned long long *status,
                          uint32_t tiles, hipStream_t s);
 uint32_t pair_sentinel(uint32_t tiles);
