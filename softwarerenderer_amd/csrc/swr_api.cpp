@@ -76,7 +76,8 @@ struct swr_context {
         vmod_out,     // rows a vertex module wrote
         zscratch[2];  // scratch of the differentiation kernels
     uint64_t prim_cap = 0, pair_cap = 0;
-    unsigned long long *status_host = nullptr;
+    unsigned long long *status_host = nullptr;  // pinned; status_map: its device address
+    unsigned long long *status_map = nullptr;
 
     bool profiling = false;
     hipEvent_t ev[S_COUNT + 1] = {};
@@ -451,10 +452,14 @@ uint32_t sort_blocks(uint64_t pair_cap)
 size_t hist_bytes(uint32_t G) { return (size_t)256 * (G + 1) * 4; }
 // kept-pair counts of the expansion chunks (256 slots at the least)
 size_t chunk_kept_bytes(uint64_t pair_cap) { return (pair_cap / 256 + 1) * 4; }
-// the expansion chunk launch_expand uses for a tuning value
-int expand_chunk_of(int tuned)
+// The expansion chunk of a draw: the tuned one, else 1024, or 256 where the pair arena is small:
+// up to 2^17 pairs make at most 128 workgroups of 1024, each a chain of four rounds of dependent
+// loads, while 512 of one round still fit the GPU at once: the VGA sphere, 9,262 pairs: 16 -> 6 us.
+int expand_chunk_of(int tuned, uint64_t pair_cap)
 {
-    return (tuned == 256 || tuned == 512 || tuned == 2048 || tuned == 4096) ? tuned : 1024;
+    if (tuned == 256 || tuned == 512 || tuned == 2048 || tuned == 4096)
+        return tuned;
+    return tuned == 0 && pair_cap <= (1u << 17) ? 256 : 1024;
 }
 
 // ---- the no-allocation draw's scratch ------------------------------------------------------
@@ -801,7 +806,7 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
                                   A.prim_cap, A.pair_cap, c->stream));
         record(c, 2);
         HIP_TRY(c, launch_geom_emit(g, c->stream));
-        HIP_TRY(c, launch_expand(g, c->stream, c->tune.expand_chunk));
+        HIP_TRY(c, launch_expand(g, c->stream, expand_chunk_of(c->tune.expand_chunk, A.pair_cap)));
         record(c, 3);
         SortBuffers sb;
         sb.keys_a = A.pk_a;
@@ -813,7 +818,8 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
         sb.ranges = A.ranges;
         sb.blocks = G;
         sb.chunk_kept = A.chunk_kept;
-        sb.chunk = (uint32_t)expand_chunk_of(c->tune.expand_chunk);
+        sb.chunk = (uint32_t)expand_chunk_of(c->tune.expand_chunk, A.pair_cap);
+        sb.out = {c->status_map, sync ? 0 : 1};
         HIP_TRY(c, sort_pairs(sb, g.status, tiles, c->stream));
         record(c, 4);
         HIP_TRY(c, launch_ranges(sb, g.status, tiles, c->stream));
@@ -858,14 +864,12 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
         // Block mode draws every triangle with Block traversal (Rasterizer.h:433-445)
         r.spans = bt ? (bt->spans ? 1 : 0) : (c->raster_mode != SWR_RASTER_BLOCK ? 1 : 0);
         r.queue = c->tune.raster_queue > 0 ? A.clipq_cnt + CLIPQ_COUNTERS : nullptr;
-        r.fold = sync ? 0 : 1;
+        r.fold = 0;  // the sort's last kernel folds and hands over the status words
         if (ps.program == SWR_PS_TEXTURE)
             r.tex = (const TexDev *)static_cast<const swr_texture *>(ps.texture)->desc.p;
         HIP_TRY(c, launch_raster(ps, L, r, c->stream, c->tune.raster_waves ? c->tune.raster_waves : 4,
                                  c->tune.raster_group));
         record(c, 6);
-        HIP_TRY(c, hipMemcpyAsync(c->status_host, c->status.p, ST_WORDS * 8, hipMemcpyDeviceToHost,
-                                  c->stream));
         if (!sync) {
             c->async_pending = true;
             return SWR_OK;
@@ -1037,6 +1041,7 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
         sb.tot = sb.hist + (size_t)256 * G;
         sb.ranges = (uint32_t *)c->ranges.p;
         sb.blocks = G;
+        sb.out = {c->status_map, 0};
         HIP_TRY(c, sort_pairs(sb, g.status, tiles, c->stream));
         record(c, 4);
         HIP_TRY(c, launch_ranges(sb, g.status, tiles, c->stream));
@@ -1071,8 +1076,6 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
         r.user = ps.uniforms;
         HIP_TRY(c, launch_lines_raster(ps, L, r, c->stream));
         record(c, 6);
-        HIP_TRY(c, hipMemcpyAsync(c->status_host, c->status.p, ST_WORDS * 8,
-                                  hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         rc = check_status(c);
         if (rc)
@@ -1195,7 +1198,13 @@ int swr_create(swr_context **out, int device)
     c->ps.checker_cells = 8.0f;
     c->vs.program = SWR_VS_DUMMY;
     if (hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void **)&c->status_host, ST_WORDS * 8, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&c->status_host, ST_WORDS * 8,
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&c->status_map, c->status_host, 0) != hipSuccess) {
+        if (c->status_host)
+            (void)hipHostFree(c->status_host);
+        if (c->own)
+            (void)hipStreamDestroy(c->own);
         delete c;
         return SWR_ERR_HIP;
     }

@@ -338,11 +338,30 @@ struct RasterArgs {
 
 // An asynchronous draw's failures, kept for the next swr_synchronize: once every earlier
 // kernel of the draw has finished (stream order), its overflow and error words are final.
-__device__ inline void fold_status(unsigned long long *st)
+// Returns the sticky word.
+__device__ inline unsigned long long fold_status(unsigned long long *st)
 {
     const unsigned long long f = (st[ST_OVERFLOW] ? 1ull : 0ull) | (st[ST_ERROR] << 1);
-    if (f)
-        atomicOr(&st[ST_STICKY], f);
+    return f ? atomicOr(&st[ST_STICKY], f) | f : st[ST_STICKY];
+}
+
+// The last kernel before the raster stage hands the status words, final by then, to the host:
+// called by the first wave of one workgroup, a word per lane.  `host` is pinned memory the GPU
+// writes in place; a copy after the raster stage would cost a launch of its own (4 us of a
+// small frame's 81).
+struct StatusOut {
+    unsigned long long *host;  // nullptr: nothing to hand over
+    int fold;                  // 1: an asynchronous draw; its failures go to ST_STICKY first
+};
+__device__ inline void hand_over_status(unsigned long long *st, const StatusOut &o)
+{
+    if (!o.host)
+        return;
+    const uint32_t lane = threadIdx.x;
+    if (lane < (uint32_t)ST_WORDS) {
+        const unsigned long long v = lane == ST_STICKY && o.fold ? fold_status(st) : st[lane];
+        __hip_atomic_store(&o.host[lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // Scene-local state of a batched draw over the single-draw arguments.

@@ -14,7 +14,7 @@
 // The vertex cache of the reference (VertexCache.h:29-63, used at VertexProcessor.cpp:86-117)
 // maps an index to an already shaded output vertex within a batch.  Vertex programs are
 // pure, so the results do not depend on which reference to a vertex shades it.  Here the
-// vertex pass (k_vertex) shades every vertex of the attribute buffer once, in index order,
+// vertex pass (shade_vertex, in the begin kernel) shades every vertex of the attribute buffer once, in index order,
 // into post-transform arrays (window-space position and clip mask), which both geometry
 // passes read by index; the emit pass fetches only the varyings the vertex program copies.
 // Triangles with a vertex outside a clip plane (clip mask != 0) re-run the program for the
@@ -946,6 +946,21 @@ fans:
     }
 }
 
+// The vertex pass: every vertex of attribute 0 shaded once (VertexProcessor.cpp:134-150 with
+// the built-in program), its clip mask (VertexProcessor.cpp:122-132) and its window-space
+// position (VertexProcessor.cpp:364-373; meaningful where the mask is 0, which is the only
+// case that reads it).
+__device__ __forceinline__ void shade_vertex(const GeomArgs &a, uint32_t v)
+{
+    Pos4 P;
+    float none[1];
+    fetch_vertex<0>(a, (int32_t)v, P, none);
+    const WinV w = to_window(a, P);
+    a.vwin[v] = make_float4(w.x, w.y, w.z, w.w);
+    a.vmask[v] = (uint8_t)clip_mask(P);
+}
+
+// Clears what a draw starts from, and runs the vertex pass (nothing it writes is cleared here).
 __global__ void __launch_bounds__(256) k_begin(GeomArgs a)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -957,6 +972,9 @@ __global__ void __launch_bounds__(256) k_begin(GeomArgs a)
         a.clipq_cnt[CLIPQ_COUNTERS + i * RASTER_QUEUE_STRIDE] = 0;
     for (uint32_t k = i; k < 2 * a.tiles; k += gridDim.x * blockDim.x)
         a.ranges[k] = 0;
+    if (a.vwin)
+        for (uint32_t v = i; v < a.nverts; v += gridDim.x * blockDim.x)
+            shade_vertex(a, v);
     // the last batch's unused (batch, phase, j) slots count nothing
     uint32_t tail = a.batches * 1024u - a.tris;
     for (uint32_t k = i; k < tail; k += gridDim.x * blockDim.x) {
@@ -965,23 +983,6 @@ __global__ void __launch_bounds__(256) k_begin(GeomArgs a)
         a.grp[(size_t)bb * 2048 + jj] = make_uint2(0, 0);
         a.grp[(size_t)bb * 2048 + 1024 + jj] = make_uint2(0, 0);
     }
-}
-
-// The vertex pass: every vertex of attribute 0 shaded once (VertexProcessor.cpp:134-150 with
-// the built-in program), its clip mask (VertexProcessor.cpp:122-132) and its window-space
-// position (VertexProcessor.cpp:364-373; meaningful where the mask is 0, which is the only
-// case that reads it).
-__global__ void __launch_bounds__(256) k_vertex(GeomArgs a)
-{
-    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= a.nverts)
-        return;
-    Pos4 P;
-    float none[1];
-    fetch_vertex<0>(a, (int32_t)v, P, none);
-    const WinV w = to_window(a, P);
-    a.vwin[v] = make_float4(w.x, w.y, w.z, w.w);
-    a.vmask[v] = (uint8_t)clip_mask(P);
 }
 
 __global__ void __launch_bounds__(256) k_geom_count(GeomArgs a)
@@ -1322,6 +1323,8 @@ static uint32_t clip_blocks(uint64_t tris)
 hipError_t launch_begin(const GeomArgs &a, hipStream_t s)
 {
     uint32_t work = 2 * a.tiles > a.batches * 1024u ? 2 * a.tiles : a.batches * 1024u;
+    if (a.vwin && a.nverts > work)
+        work = a.nverts;
     uint32_t blocks = (work + 255) / 256;
     if (blocks > 2048) blocks = 2048;
     if (blocks < 1) blocks = 1;
@@ -1333,8 +1336,6 @@ hipError_t launch_geom_count(const GeomArgs &a, hipStream_t s)
 {
     if (!a.tris)
         return hipSuccess;
-    if (a.vwin && a.nverts)
-        hipLaunchKernelGGL(k_vertex, dim3((a.nverts + 255) / 256), dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_geom_count, dim3((a.tris + 255) / 256), dim3(256), 0, s, a);
     if (!a.window_input)
         hipLaunchKernelGGL(k_clip_count, dim3(clip_blocks(a.tris)), dim3(CLIPQ_THREADS), 0, s, a);
@@ -1353,7 +1354,7 @@ static hipError_t launch_expand_ch(const GeomArgs &a, hipStream_t s)
 
 hipError_t launch_expand(const GeomArgs &a, hipStream_t s, int chunk)
 {
-    switch (chunk) {  // the chunk sizes swr_api.cpp's expand_chunk_of names
+    switch (chunk) {  // the chunk sizes swr_api.cpp's expand_chunk_of gives
     case 256: return launch_expand_ch<256>(a, s);
     case 512: return launch_expand_ch<512>(a, s);
     case 2048: return launch_expand_ch<2048>(a, s);

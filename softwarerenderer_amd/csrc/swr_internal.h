@@ -14,6 +14,7 @@ struct SortBuffers {
     uint32_t chunk = 0;                    // slots per expansion chunk
     uint32_t *sorted_keys, *sorted_vals;  // set by sort_pairs (the keys unless `ranged`)
     bool ranged = false;                  // sort_pairs wrote the tiles' ranges itself
+    StatusOut out = {nullptr, 0};         // where the last kernel hands the status words
 };
 
 // geometry (swr_geometry.hip)
@@ -57,8 +58,8 @@ hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uin
                                unsigned long long *status, uint64_t cap_prims,
                                uint64_t cap_pairs, hipStream_t s);
 hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tiles, hipStream_t s);
-hipError_t launch_ranges(const SortBuffers &sb, const unsigned long long *status,
-                         uint32_t tiles, hipStream_t s);
+hipError_t launch_ranges(const SortBuffers &sb, unsigned long long *status, uint32_t tiles,
+                         hipStream_t s);
 uint32_t pair_sentinel(uint32_t tiles);
 
 // context access for the kernel files' own entry points (swr_api.cpp)

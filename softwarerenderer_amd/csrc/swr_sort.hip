@@ -623,13 +623,14 @@ __global__ void __launch_bounds__(RADIX_THREADS) k_radix_scatter(
 // pairs or not.  Runs differ in length with the picture, neighbouring tiles lie in different
 // buckets.
 __global__ void __launch_bounds__(1024) k_bucket(const uint32_t *keys, const uint32_t *vals,
-                                                 uint32_t *ovals,
-                                                 const unsigned long long *status,
+                                                 uint32_t *ovals, unsigned long long *status,
                                                  const uint32_t *tot, int bits, uint32_t tiles,
-                                                 uint32_t *ranges)
+                                                 uint32_t *ranges, StatusOut out)
 {
     extern __shared__ uint32_t s_cnt[];  // [waves][1 << bits]
     __shared__ uint32_t s_w[16];
+    if (blockIdx.x == 0 && threadIdx.x < 64)
+        hand_over_status(status, out);
     if (status[ST_OVERFLOW] | status[ST_ERROR])
         return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6, W = blockDim.x >> 6;
@@ -729,9 +730,11 @@ __global__ void __launch_bounds__(1024) k_bucket(const uint32_t *keys, const uin
 
 // Per-tile [begin, end) into the sorted kept pairs; tiles without pairs keep the zeros the
 // begin kernel wrote.
-__global__ void __launch_bounds__(256) k_ranges(const uint32_t *keys,
-                                              const unsigned long long *status, uint32_t *ranges)
+__global__ void __launch_bounds__(256) k_ranges(const uint32_t *keys, unsigned long long *status,
+                                              uint32_t *ranges, StatusOut out)
 {
+    if (blockIdx.x == 0 && threadIdx.x < 64)
+        hand_over_status(status, out);
     uint64_t m = pair_count(status, ST_KEPT);
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
          i += (uint64_t)gridDim.x * blockDim.x) {
@@ -792,7 +795,7 @@ hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tile
         uint32_t waves = sb.blocks > SCAN_ROWS ? 16 : 4;
         waves = waves < most ? waves : most;
         hipLaunchKernelGGL(k_bucket, dim3(256), dim3(64 * waves), (4u * waves) << high, s, ka, va,
-                           vb, status, sb.tot, high, tiles, sb.ranges);
+                           vb, status, sb.tot, high, tiles, sb.ranges, sb.out);
         std::swap(va, vb);
     }
     sb.sorted_keys = ka;
@@ -800,13 +803,14 @@ hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tile
     return hipGetLastError();
 }
 
-hipError_t launch_ranges(const SortBuffers &sb, const unsigned long long *status,
-                         uint32_t tiles, hipStream_t s)
+hipError_t launch_ranges(const SortBuffers &sb, unsigned long long *status, uint32_t tiles,
+                         hipStream_t s)
 {
     (void)tiles;
     if (sb.ranged)
         return hipSuccess;
-    hipLaunchKernelGGL(k_ranges, dim3(1024), dim3(256), 0, s, sb.sorted_keys, status, sb.ranges);
+    hipLaunchKernelGGL(k_ranges, dim3(1024), dim3(256), 0, s, sb.sorted_keys, status, sb.ranges,
+                       sb.out);
     return hipGetLastError();
 }
 
