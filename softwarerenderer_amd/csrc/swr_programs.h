@@ -46,44 +46,66 @@ struct ChainPixel {
     __device__ float p_raw(int k) const { return v[L::P + k]; }
     __device__ static float w_of(float raw) { return 1.0f / raw; }
     __device__ static float pvar_of(float raw, float w) { return raw * w; }
-    // a fragment's planes can be chained again at its pixel (chain_at)
+    // a fragment's planes can be chained again at its pixel (chain_planes)
     static constexpr bool REPLAY = true;
 };
 
-// Plane p of a primitive record at pixel (x, y) by the chain the raster kernel runs, in the
-// same operations: Block (PixelShaderBase.h:55-94): init at the 8x8 block's first pixel
-// centre, +b per row, +a per column; Span (PixelShaderBase.h:96-112): init at the span's
+// Planes p .. p + K - 1 of a primitive record at pixel (x, y) by the chain the raster kernel
+// runs, in the same operations: Block (PixelShaderBase.h:55-94): init at the 8x8 block's first
+// pixel centre, +b per row, +a per column; Span (PixelShaderBase.h:96-112): init at the span's
 // first pixel xl of row y, +a per pixel after it.  (x, y) must be a pixel the primitive
 // covers (for Span, xl <= x).
 // SPANS = false: the record is known to be a Block primitive.
-template <bool SPANS = true>
-__device__ inline float chain_at(const float *rec, int p, int x, int y, int sc_minx, int sc_maxx)
+//
+// Lanes are pixels of different primitives, so nothing is shared between them; the K chains
+// step together under one lane mask per step (K additions where a chain by itself takes an
+// addition and a select, or a loop of its own): the store stage of a block with few primitives
+// is most of its work (48 spheres, 3.6 primitives per block: raster 328 -> 280 us).
+template <int K, bool SPANS = true>
+__device__ inline void chain_planes(const float *rec, int p, int x, int y, int sc_minx,
+                                    int sc_maxx, float (&v)[K])
 {
-    const float pa = rec[REC_PARAM + 3 * p], pb = rec[REC_PARAM + 3 * p + 1],
-                pc = rec[REC_PARAM + 3 * p + 2];
-    const uint32_t flags = __float_as_uint(rec[REC_FLAGS]);
-    if (!SPANS || (flags & FLAG_BLOCK)) {
-        // y - by additions of b, then x - bx of a (0..7 each), as selects from the running
-        // sums: no per-lane trip counts
-        const int bx = x & ~(TILE - 1), by = y & ~(TILE - 1);
-        const int dy = y - by, dx = x - bx;
-        float r = pa * ((float)bx + 0.5f) + pb * ((float)by + 0.5f) + pc, t = r;
+    float pa[K], pb[K], pc[K];
 #pragma unroll
-        for (int k = 1; k < TILE; ++k) {
-            t = t + pb;
-            r = k <= dy ? t : r;
-        }
-        t = r;
-#pragma unroll
-        for (int i = 1; i < TILE; ++i) {
-            t = t + pa;
-            r = i <= dx ? t : r;
-        }
-        return r;
+    for (int k = 0; k < K; ++k) {
+        pa[k] = rec[REC_PARAM + 3 * (p + k)];
+        pb[k] = rec[REC_PARAM + 3 * (p + k) + 1];
+        pc[k] = rec[REC_PARAM + 3 * (p + k) + 2];
     }
-    int xl = 0, xr = 0;
-    span_row_extent(rec, flags, y, sc_minx, sc_maxx, xl, xr);
-    return chain_add(pa * ((float)xl + 0.5f) + pb * ((float)y + 0.5f) + pc, pa, x - xl);
+    // first pixel, rows to step down, columns to step right
+    int x0 = x & ~(TILE - 1), y0 = y & ~(TILE - 1);
+    int ny = y - y0, nx = x - x0;
+    if constexpr (SPANS) {
+        const uint32_t flags = __float_as_uint(rec[REC_FLAGS]);
+        if (!(flags & FLAG_BLOCK)) {
+            int xl = 0, xr = 0;
+            span_row_extent(rec, flags, y, sc_minx, sc_maxx, xl, xr);
+            x0 = xl;
+            y0 = y;
+            ny = 0;
+            nx = x - xl;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        v[k] = pa[k] * ((float)x0 + 0.5f) + pb[k] * ((float)y0 + 0.5f) + pc[k];
+    for (int n = 0; n < ny; ++n) {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            v[k] = v[k] + pb[k];
+    }
+    // a Span pixel far from its span's start: the additions fast-forwarded
+    if (SPANS && nx > 16) {
+#pragma unroll 1
+        for (int k = 0; k < K; ++k)
+            v[k] = chain_add(v[k], pa[k], nx);
+    } else {
+        for (int n = 0; n < nx; ++n) {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                v[k] = v[k] + pa[k];
+        }
+    }
 }
 
 // ---- pixel programs (include/swr_hip.h) ---------------------------------------------------
@@ -110,7 +132,7 @@ struct ProgCoverage {
 // RasterizerTest.cpp:38-48.  Every fragment overwrites the pixel, so only the last one
 // counts: for triangles the raster kernel walks the block's list from its end (LAST_WINS),
 // shade keeps the record of the first fragment met there (the kernel chains nothing, CHAINED)
-// and store chains its colour planes at the pixel (chain_at) and packs them once.
+// and store chains its colour planes at the pixel (chain_planes) and packs them once.
 template <class L>
 struct ProgRGB {
     static constexpr int KEY_WORD = REC_KEY;
@@ -148,9 +170,9 @@ struct ProgRGB {
         uint32_t c = s.c;
         if constexpr (PX::REPLAY) {
             const float *rec = a.prims + (size_t)s.prim * (size_t)a.stride;
-            c = pack(chain_at<PX::SPANS>(rec, L::A, x, y, a.sc_minx, a.sc_maxx),
-                     chain_at<PX::SPANS>(rec, L::A + 1, x, y, a.sc_minx, a.sc_maxx),
-                     chain_at<PX::SPANS>(rec, L::A + 2, x, y, a.sc_minx, a.sc_maxx));
+            float v[3];
+            chain_planes<3, PX::SPANS>(rec, L::A, x, y, a.sc_minx, a.sc_maxx, v);
+            c = pack(v[0], v[1], v[2]);
         }
         static_cast<uint32_t *>(a.t0)[o] = c;
     }
@@ -159,7 +181,7 @@ struct ProgRGB {
 // Only the last depth-passing fragment of a pixel reaches the targets, and its colour is a
 // pure function of its interpolants.  So shade keeps only that fragment: for triangles its
 // primitive record (the raster kernel chains z alone, CHAINED), and store chains its other
-// planes again at the pixel (chain_at: the same operations on the same values); for points
+// planes again at the pixel (chain_planes: the same operations on the same values); for points
 // and lines its raw values.  Store computes the colour once.
 template <class L>
 struct ProgDepthChecker {
@@ -200,13 +222,16 @@ struct ProgDepthChecker {
         if (s0.hit) {
             State s = s0;
             if constexpr (PX::REPLAY) {
+                static_assert(L::A == L::IW + 1 && L::P == L::IW + 4, "planes 1/w, avar, pvar");
                 const float *rec = a.prims + (size_t)s.prim * (size_t)a.stride;
-                s.wr = chain_at<PX::SPANS>(rec, L::IW, x, y, a.sc_minx, a.sc_maxx);
-                s.a0 = chain_at<PX::SPANS>(rec, L::A, x, y, a.sc_minx, a.sc_maxx);
-                s.a1 = chain_at<PX::SPANS>(rec, L::A + 1, x, y, a.sc_minx, a.sc_maxx);
-                s.a2 = chain_at<PX::SPANS>(rec, L::A + 2, x, y, a.sc_minx, a.sc_maxx);
-                s.p0 = chain_at<PX::SPANS>(rec, L::P, x, y, a.sc_minx, a.sc_maxx);
-                s.p1 = chain_at<PX::SPANS>(rec, L::P + 1, x, y, a.sc_minx, a.sc_maxx);
+                float v[6];
+                chain_planes<6, PX::SPANS>(rec, L::IW, x, y, a.sc_minx, a.sc_maxx, v);
+                s.wr = v[0];
+                s.a0 = v[1];
+                s.a1 = v[2];
+                s.a2 = v[3];
+                s.p0 = v[4];
+                s.p1 = v[5];
             }
             const float w = PX::w_of(s.wr);  // only the depth-passing pixels read pvar
             const float u = PX::pvar_of(s.p0, w), t = PX::pvar_of(s.p1, w);
@@ -497,7 +522,7 @@ struct ProgTexture {
     static constexpr bool PLANES = true;
     // every fragment overwrites the pixel: shade keeps the last one's record (the raster
     // kernel walks the list from its end) and store samples once, from the planes chained
-    // again at the pixel (chain_at)
+    // again at the pixel (chain_planes)
     static constexpr int CHAINED = 0;
     static constexpr bool LAST_WINS = true;
     struct State { uint32_t prim; bool hit; };
@@ -526,11 +551,11 @@ struct ProgTexture {
         if (!s.hit)
             return;
         const float *rec = a.prims + (size_t)s.prim * (size_t)a.stride;
-        const float w = PX::w_of(chain_at<PX::SPANS>(rec, L::IW, x, y, a.sc_minx, a.sc_maxx));
-        const float u =
-            PX::pvar_of(chain_at<PX::SPANS>(rec, L::P, x, y, a.sc_minx, a.sc_maxx), w);
-        const float t =
-            PX::pvar_of(chain_at<PX::SPANS>(rec, L::P + 1, x, y, a.sc_minx, a.sc_maxx), w);
+        static_assert(L::P == L::IW + 1, "planes 1/w, pvar");
+        float c[3];
+        chain_planes<3, PX::SPANS>(rec, L::IW, x, y, a.sc_minx, a.sc_maxx, c);
+        const float w = PX::w_of(c[0]);
+        const float u = PX::pvar_of(c[1], w), t = PX::pvar_of(c[2], w);
         const float *P = rec + REC_PARAM;
         const float xf = (float)x + 0.5f, yf = (float)y + 0.5f;
         float dudx, dudy, dvdx, dvdy;

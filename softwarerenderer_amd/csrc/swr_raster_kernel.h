@@ -433,7 +433,8 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
 #pragma unroll
                     for (int k = 0; k < K; ++k)
                         r[k] = pa[k] * xf + pb[k] * yf + pc[k];
-                    row_starts(r, pb);
+                    if (!SPANS || __ballot(act && blk) != 0ull)
+                        row_starts(r, pb);
 #pragma unroll
                     for (int k = 0; k < K; ++k) {
                         if constexpr (SPANS)
