@@ -428,15 +428,32 @@ __device__ inline float tex_log2(float xf)
     return (float)((double)e + ln_m * 1.4426950408889634074);
 }
 
-// sampleBilinear + bilinearLerpColors, Texture.h:148-228
-__device__ inline uint32_t tex_bilinear(const TexDev &t, int lv, float u, float v)
+// A mip level, and the two of a level of detail with the blend between them: the same for all
+// taps of a pixel, so the tables are read and log2 taken once and a tap's loads wait for
+// nothing but its coordinates.
+struct TexLevel {
+    const uint32_t *p;
+    int w, h;
+};
+struct TexLod {
+    TexLevel base, next;
+    bool same;
+    float frac;
+};
+__device__ inline TexLevel tex_level(const TexDev &t, int lv)
 {
-    const int w = t.w[lv], h = t.h[lv];
+    return {t.texels + t.off[lv], t.w[lv], t.h[lv]};
+}
+
+// sampleBilinear + bilinearLerpColors, Texture.h:148-228
+__device__ inline uint32_t tex_bilinear(const TexLevel &t, float u, float v)
+{
+    const int w = t.w, h = t.h;
     const float px = u * (float)(w - 1), py = v * (float)(h - 1);
     const int x0 = imax(0, f2i(floorf(px))), y0 = imax(0, f2i(floorf(py)));
     const int x1 = tex_imin(w - 1, x0 + 1), y1 = tex_imin(h - 1, y0 + 1);
     const float fx = px - (float)x0, fy = py - (float)y0;
-    const uint32_t *p = t.texels + t.off[lv];
+    const uint32_t *p = t.p;
     const uint32_t c00 = p[(size_t)y0 * w + x0], c10 = p[(size_t)y0 * w + x1];
     const uint32_t c01 = p[(size_t)y1 * w + x0], c11 = p[(size_t)y1 * w + x1];
     uint32_t out[3];
@@ -450,23 +467,29 @@ __device__ inline uint32_t tex_bilinear(const TexDev &t, int lv, float u, float 
     return tex_pack(out[0], out[1], out[2]);
 }
 
-// sampleTrilinear + lerpColors, Texture.h:121-146, 200-205
-__device__ inline uint32_t tex_trilinear(const TexDev &t, float u, float v, float rho)
+// sampleTrilinear's level of detail, Texture.h:121-133
+__device__ inline TexLod tex_lod(const TexDev &t, float rho)
 {
     float lod = tex_log2(rho < 1e-6f ? 1e-6f : rho);
     lod = tex_clamp(lod, 0.0f, (float)(t.levels - 1));
     const int base = f2i(floorf(lod));
     const int next = tex_imin(base + 1, t.levels - 1);
-    const float frac = tex_clamp(lod - (float)base, 0.0f, 1.0f);
-    const uint32_t cb = tex_bilinear(t, base, u, v);
-    if (base == next)
+    return {tex_level(t, base), tex_level(t, next), base == next,
+            tex_clamp(lod - (float)base, 0.0f, 1.0f)};
+}
+
+// sampleTrilinear + lerpColors, Texture.h:133-146, 200-205
+__device__ inline uint32_t tex_trilinear(const TexLod &l, float u, float v)
+{
+    const uint32_t cb = tex_bilinear(l.base, u, v);
+    if (l.same)
         return cb;
-    const uint32_t cn = tex_bilinear(t, next, u, v);
+    const uint32_t cn = tex_bilinear(l.next, u, v);
     uint32_t out[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const int d = (int)tex_ch(cn, k) - (int)tex_ch(cb, k);
-        const uint8_t step = (uint8_t)f2i((float)d * frac);
+        const uint8_t step = (uint8_t)f2i((float)d * l.frac);
         out[k] = (uint8_t)(tex_ch(cb, k) + step);
     }
     return tex_pack(out[0], out[1], out[2]);
@@ -488,7 +511,7 @@ __device__ inline uint32_t tex_sample(const TexDev &t, float u, float v, float d
     const float ratio = ref_min(major / minor, (float)t.max_aniso);
     const int n = imax(1, f2i(ceilf(ratio)));
     if (n <= 1)
-        return tex_trilinear(t, u, v, major);
+        return tex_trilinear(tex_lod(t, major), u, v);
     float mdu, mdv;
     if (dx_len > dy_len) {
         mdu = dudx / dx_len;
@@ -499,11 +522,13 @@ __device__ inline uint32_t tex_sample(const TexDev &t, float u, float v, float d
     }
     float r = 0, g = 0, b = 0;
     const float step = 1.0f / (float)n;
+    const TexLod lod = tex_lod(t, minor);
+#pragma unroll 2
     for (int i = 0; i < n; ++i) {
         const float tt = ((float)i + 0.5f) * step - 0.5f;
         const float su = tex_wrap(u + mdu * major * tt);
         const float sv = tex_wrap(v + mdv * major * tt);
-        const uint32_t c = tex_trilinear(t, su, sv, minor);
+        const uint32_t c = tex_trilinear(lod, su, sv);
         r += (float)tex_ch(c, 0);
         g += (float)tex_ch(c, 1);
         b += (float)tex_ch(c, 2);
