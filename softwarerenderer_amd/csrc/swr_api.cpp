@@ -947,9 +947,10 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
     if (rc)
         return rc;
 
-    HIP_TRY(c, ensure(c, c->app, P * 4));
-    HIP_TRY(c, ensure(c, c->app_ex, P * 4));
-    HIP_TRY(c, ensure(c, c->scan_tmp, scan_tmp_elems(P) * 8));
+    HIP_TRY(c, ensure(c, c->app, P * 8));
+    HIP_TRY(c, ensure(c, c->app_ex, P * 8));
+    // the scan's block sums, then the count workgroups' totals
+    HIP_TRY(c, ensure(c, c->scan_tmp, (scan_tmp_elems(P) + lines_groups(P)) * 8));
     HIP_TRY(c, ensure(c, c->ranges, (size_t)tiles * 8));
     HIP_TRY(c, ensure(c, c->status, ST_WORDS * 8));
 
@@ -994,14 +995,16 @@ int draw_lines_points(swr_context *c, int mode, const int32_t *indices, size_t c
     A.prims = P;
     A.iz = ps.interpolate_z ? 1 : 0;
     A.iw = ps.interpolate_w ? 1 : 0;
-    A.count = (uint32_t *)c->app.p;
-    A.first = (const uint32_t *)c->app_ex.p;
+    A.count = (uint2 *)c->app.p;
+    A.first = (const uint2 *)c->app_ex.p;
+    A.parts = (unsigned long long *)c->scan_tmp.p + scan_tmp_elems(P);
     A.fstride = fragment_stride(L);
 
     record(c, 0);
     HIP_TRY(c, launch_lines_count(A, c->stream));
     record(c, 1);
-    HIP_TRY(c, scan_u32(A.count, (uint32_t *)c->app_ex.p, P, (uint32_t *)c->scan_tmp.p, c->stream));
+    HIP_TRY(c, scan_lines(A.count, (uint2 *)c->app_ex.p, P, (uint2 *)c->scan_tmp.p, A.parts,
+                          lines_groups(P), g.status, c->stream));
     record(c, 2);
     HIP_TRY(c, hipMemcpyAsync(c->status_host, c->status.p, ST_WORDS * 8, hipMemcpyDeviceToHost,
                               c->stream));

@@ -32,13 +32,15 @@ struct LineArgs {
     int mode;               // SWR_DRAW_POINT or SWR_DRAW_LINE
     uint64_t prims;         // primitives: index pairs (lines) or indices (points)
     int iz, iw;             // InterpolateZ / InterpolateW: which values the DDA steps
-    uint32_t *count;        // [prims] fragments of each primitive (count pass)
-    const uint32_t *first;  // [prims] exclusive scan of count
+    uint2 *count;           // [prims] (drawn, fragments) of each primitive (count pass)
+    const uint2 *first;     // [prims] exclusive scan of count
+    unsigned long long *parts;  // [lines_groups(prims)] fragments per count workgroup
     float *frags;           // fragment records (emit pass)
     int fstride;            // words per fragment record
     uint32_t *keys, *vals;  // (tile, fragment) pairs in fragment order
 };
 int fragment_stride(const ParamLayout &L);
+uint32_t lines_groups(uint64_t prims);
 hipError_t launch_lines_count(const LineArgs &a, hipStream_t s);
 hipError_t launch_lines_emit(const LineArgs &a, hipStream_t s);
 hipError_t launch_lines_raster(const swr_pixel_shader_desc &ps, const ParamLayout &L,
@@ -46,7 +48,11 @@ hipError_t launch_lines_raster(const swr_pixel_shader_desc &ps, const ParamLayou
 
 // scans and sort (swr_sort.hip)
 uint64_t scan_tmp_elems(uint64_t n);
-hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *tmp, hipStream_t s);
+// the (drawn, fragments) scan of points and lines; status[ST_PRIMS] gets the drawn total and
+// status[ST_PAIRS] the 64-bit sum of the nparts parts (all the fragments)
+hipError_t scan_lines(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
+                      const unsigned long long *parts, uint32_t nparts,
+                      unsigned long long *status, hipStream_t s);
 hipError_t scan_pairs(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
                       unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
                       hipStream_t s);

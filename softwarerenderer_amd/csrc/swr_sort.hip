@@ -159,15 +159,9 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(T *sums, uint32_t nb
     }
 }
 
-// The total of the scan, published by the thread that owns the last element: a u32 scan
-// writes it to status[word]; the (prims, pairs) scan writes both totals and flags arena
-// overflow against the capacities.
-__device__ inline void publish_totals(uint32_t t, unsigned long long *status, int word, uint64_t,
-                                      uint64_t)
-{
-    status[word] = t;
-}
-__device__ inline void publish_totals(uint2 t, unsigned long long *status, int, uint64_t cap_x,
+// The totals of the (prims, pairs) scan, published by the thread that owns the last element,
+// with arena overflow against the capacities.
+__device__ inline void publish_totals(uint2 t, unsigned long long *status, uint64_t cap_x,
                                       uint64_t cap_y)
 {
     status[ST_PRIMS] = t.x;
@@ -200,7 +194,7 @@ __device__ T block_carry(const T *sums, uint32_t b)
 // live total goes to status[ST_LIVE].
 template <typename T, bool CARRY>
 __device__ void down_tile(const T *in, uint64_t n, const T *sums, T *out,
-                          unsigned long long *status, int word, uint64_t cap_x, uint64_t cap_y,
+                          unsigned long long *status, uint64_t cap_x, uint64_t cap_y,
                           uint32_t b, uint32_t *list = nullptr)
 {
     const T carry = CARRY ? block_carry<T>(sums, b) : sums[b];
@@ -226,7 +220,7 @@ __device__ void down_tile(const T *in, uint64_t n, const T *sums, T *out,
             }
         }
         if (status && !list && base + i == n - 1)
-            publish_totals(sadd(run, vals[i]), status, word, cap_x, cap_y);
+            publish_totals(sadd(run, vals[i]), status, cap_x, cap_y);
         run = sadd(run, vals[i]);
     }
     store_items<T>(out, base, n, o);
@@ -235,11 +229,11 @@ __device__ void down_tile(const T *in, uint64_t n, const T *sums, T *out,
 template <typename T, bool CARRY>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_down(const T *in, uint64_t n,
                                                           const T *sums, T *out,
-                                                          unsigned long long *status, int word,
+                                                          unsigned long long *status,
                                                           uint64_t cap_x, uint64_t cap_y,
                                                           uint32_t *list)
 {
-    down_tile<T, CARRY>(in, n, sums, out, status, word, cap_x, cap_y, blockIdx.x, list);
+    down_tile<T, CARRY>(in, n, sums, out, status, cap_x, cap_y, blockIdx.x, list);
 }
 
 // The per-triangle (appended fans, live) counts and the per-slot (primitives, pairs) counts
@@ -261,9 +255,9 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_down2(
     uint64_t cap_x, uint64_t cap_y)
 {
     if (blockIdx.x < nba)
-        down_tile<uint2, true>(a, na, sa, oa, status, 0, 0, 0, blockIdx.x, list);
+        down_tile<uint2, true>(a, na, sa, oa, status, 0, 0, blockIdx.x, list);
     else
-        down_tile<uint2, true>(g, ng, sg, og, status, 0, cap_x, cap_y, blockIdx.x - nba);
+        down_tile<uint2, true>(g, ng, sg, og, status, cap_x, cap_y, blockIdx.x - nba);
 }
 
 // Scans of up to this many blocks skip the pass over the block sums: each block of the
@@ -273,7 +267,7 @@ constexpr uint32_t SCAN_CARRY_BLOCKS = 8192;
 
 template <typename T>
 hipError_t scan_impl(const T *in, T *out, uint64_t n, T *tmp, unsigned long long *status,
-                     int word, uint64_t cap_x, uint64_t cap_y, hipStream_t s,
+                     uint64_t cap_x, uint64_t cap_y, hipStream_t s,
                      uint32_t *list = nullptr)
 {
     if (!n)
@@ -282,27 +276,55 @@ hipError_t scan_impl(const T *in, T *out, uint64_t n, T *tmp, unsigned long long
     hipLaunchKernelGGL(k_scan_reduce<T>, dim3(nb), dim3(SCAN_THREADS), 0, s, in, n, tmp);
     if (nb <= SCAN_CARRY_BLOCKS) {
         hipLaunchKernelGGL((k_scan_down<T, true>), dim3(nb), dim3(SCAN_THREADS), 0, s, in, n,
-                           tmp, out, status, word, cap_x, cap_y, list);
+                           tmp, out, status, cap_x, cap_y, list);
     } else {
         hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nb);
         hipLaunchKernelGGL((k_scan_down<T, false>), dim3(nb), dim3(SCAN_THREADS), 0, s, in, n,
-                           tmp, out, status, word, cap_x, cap_y, list);
+                           tmp, out, status, cap_x, cap_y, list);
     }
     return hipGetLastError();
 }
 
 uint64_t scan_tmp_elems(uint64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
 
-hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *tmp, hipStream_t s)
+__global__ void __launch_bounds__(SCAN_THREADS) k_sum_parts(const unsigned long long *parts,
+                                                            uint32_t n,
+                                                            unsigned long long *status)
 {
-    return scan_impl<uint32_t>(in, out, n, tmp, nullptr, 0, 0, 0, s);
+    __shared__ unsigned long long s_w[SCAN_THREADS / 64];
+    unsigned long long x = 0;
+    for (uint32_t k = threadIdx.x; k < n; k += SCAN_THREADS)
+        x += parts[k];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1)
+        x += __shfl_xor(x, o, 64);
+    if ((threadIdx.x & 63u) == 0)
+        s_w[threadIdx.x >> 6] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < SCAN_THREADS / 64; ++w)
+            x += s_w[w];
+        status[ST_PAIRS] = x;
+    }
+}
+
+hipError_t scan_lines(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
+                      const unsigned long long *parts, uint32_t nparts,
+                      unsigned long long *status, hipStream_t s)
+{
+    // (the capacities of lines and points are the host's business: no overflow here)
+    hipError_t e = scan_impl<uint2>(in, out, n, tmp, status, ~0ull, ~0ull, s);
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(SCAN_THREADS), 0, s, parts, nparts, status);
+    return hipGetLastError();
 }
 
 hipError_t scan_pairs(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
                       unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
                       hipStream_t s)
 {
-    return scan_impl<uint2>(in, out, n, tmp, status, 0, cap_prims, cap_pairs, s);
+    return scan_impl<uint2>(in, out, n, tmp, status, cap_prims, cap_pairs, s);
 }
 
 hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uint32_t *live,
@@ -316,7 +338,7 @@ hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uin
     uint2 *sa = static_cast<uint2 *>(tmp);
     uint2 *sg = sa + scan_tmp_elems(na);
     if (!na || !ng || nba > SCAN_CARRY_BLOCKS || nbg > SCAN_CARRY_BLOCKS) {
-        hipError_t e = scan_impl<uint2>(app, app_ex, na, sa, status, 0, 0, 0, s, live);
+        hipError_t e = scan_impl<uint2>(app, app_ex, na, sa, status, 0, 0, s, live);
         if (e != hipSuccess)
             return e;
         return scan_pairs(grp, grp_ex, ng, sg, status, cap_prims, cap_pairs, s);

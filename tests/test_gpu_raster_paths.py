@@ -86,3 +86,24 @@ def test_chained_planes(gpu, cpu_oracle, prog, shape, n):
         assert_same(run_cpu(cpu_oracle, pipe, sc), run_gpu(pipe, sc, rasterizer=r),
                     f"n={n} mode={mode} {GROUPS[shape]} {prog}")
         r.close()
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 65, 150])
+@pytest.mark.parametrize("prog", [(O.PS_LOG, 3, 2), (O.PS_LOG, 16, 16), (O.PS_DEPTH_CHECKER, 3, 2)])
+def test_lines_of_all_lengths(gpu, cpu_oracle, prog, n):
+    """Lines of 0 to some 2,000 steps side by side, many of them partly off the target: their
+    pieces (64 steps) start where the step-by-step walk would be."""
+    w, h = 700, 45
+    v = scenes.window_lines(n, 11 + n, w, h, long_frac=0.0)
+    rng = np.random.default_rng(n)
+    steps = np.resize([0, 1, 63, 64, 65, 128, 129, 700, 2000, 333], n)
+    x0 = rng.uniform(-300, 500, n)
+    v["x"][0::2], v["x"][1::2] = x0, x0 + steps * rng.choice([-1, 1], n)
+    v["y"][0::2] = rng.uniform(0, h, n)
+    v["y"][1::2] = v["y"][0::2] + rng.uniform(-1, 1, n) * np.minimum(steps, 60)
+    pipe = O.Pipeline(w, h, ps_program=prog[0], ps_z=True, ps_w=True, ps_a=prog[1], ps_p=prog[2])
+    idx = np.arange(2 * n, dtype=np.int32)
+    cap = 200_000 if prog[0] == O.PS_LOG else 0
+    assert_same(run_cpu(cpu_oracle, pipe, vertices=v, indices=idx, prim="line", log_capacity=cap),
+                run_gpu(pipe, vertices=v, indices=idx, prim="line", log_capacity=cap),
+                f"n={n} {prog}")
