@@ -92,7 +92,7 @@ def test_chained_planes(gpu, cpu_oracle, prog, shape, n):
 @pytest.mark.parametrize("prog", [(O.PS_LOG, 3, 2), (O.PS_LOG, 16, 16), (O.PS_DEPTH_CHECKER, 3, 2)])
 def test_lines_of_all_lengths(gpu, cpu_oracle, prog, n):
     """Lines of 0 to some 2,000 steps side by side, many of them partly off the target: their
-    pieces (64 steps) start where the step-by-step walk would be."""
+    pieces (32 steps) start where the step-by-step walk would be."""
     w, h = 700, 45
     v = scenes.window_lines(n, 11 + n, w, h, long_frac=0.0)
     rng = np.random.default_rng(n)
@@ -107,3 +107,38 @@ def test_lines_of_all_lengths(gpu, cpu_oracle, prog, n):
     assert_same(run_cpu(cpu_oracle, pipe, vertices=v, indices=idx, prim="line", log_capacity=cap),
                 run_gpu(pipe, vertices=v, indices=idx, prim="line", log_capacity=cap),
                 f"n={n} {prog}")
+
+
+@pytest.mark.parametrize("scissor", [(0, 0, 70, 45), (-400, -9, 480, 60), (5, 3, 50, 40)])
+@pytest.mark.parametrize("shape", [2, 3, 4])
+@pytest.mark.parametrize("prog", [(O.PS_DEPTH_CHECKER, 3, 2), (O.PS_VISIBILITY, 0, 0)])
+def test_hidden_primitives(gpu, cpu_oracle, prog, shape, scissor):
+    """Long lists of larger bins, where what lies behind a block's pixels is dropped: sloped
+    planes crossing each other, and the same planes again one unit in the last place nearer or
+    farther, in front, behind and in random order."""
+    from softwarerenderer_amd import api
+    n = 500
+    lay = _layers(n, 500 + shape, 0.5).vertices.reshape(n, 3, 6)
+    lay[:, :, 0:2] = np.clip(lay[:, :, 0:2] * 3, -0.99, 0.99)
+    same = lay.copy()
+    same[:, :, 2] = np.nextafter(same[:, :, 2], np.float32(-1) ** np.arange(n)[:, None] * 2,
+                                 dtype=np.float32)
+    v = np.concatenate([lay, same])
+    order = np.argsort(v[:, :, 2].max(1), kind="stable")
+    for mode in (O.RASTER_SPAN, O.RASTER_BLOCK, O.RASTER_ADAPTIVE):
+        for name, o in (("near first", order), ("far first", order[::-1]),
+                        ("mixed", np.random.default_rng(mode).permutation(2 * n))):
+            t = v[o].reshape(-1, 6)
+            w = np.ones((t.shape[0], 1), np.float32)
+            t = np.concatenate([t[:, :3], w, t[:, 3:], t[:, :2]], 1).astype(np.float32)
+            sc = scenes.Scene(t, np.arange(6 * n, dtype=np.int32), np.eye(4, dtype=np.float32),
+                              0, 0)
+            pipe = O.Pipeline(70, 45, raster_mode=mode, cull_mode=O.CULL_NONE, scissor=scissor,
+                              vs_program=O.VS_RAW, vs_counts=(1, 3, 2), ps_program=prog[0],
+                              ps_w=prog[0] != O.PS_VISIBILITY, ps_a=prog[1], ps_p=prog[2])
+            r = api.Rasterizer(0)
+            r.setTuning(**SHAPES[shape])
+            a, b = run_cpu(cpu_oracle, pipe, sc), run_gpu(pipe, sc, rasterizer=r)
+            r.close()
+            assert int((a.t0 != 0).sum()) > 500
+            assert_same(a, b, f"{name} mode={mode} {prog} {SHAPES[shape]}")
