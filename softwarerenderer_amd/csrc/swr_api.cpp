@@ -66,7 +66,7 @@ struct swr_context {
     } attr[SWR_MAX_VERTEX_ATTRIBS];
 
     // arenas
-    DevBuf idx, attr0, wverts, app, app_ex, live, grp, grp_ex, scan_tmp, prims, pk_a, pv_a, pk_b, pv_b,
+    DevBuf idx, attr0, wverts, app, app_ex, live, cnt, cflag, ex, scan_tmp, prims, pk_a, pv_a, pk_b, pv_b,
         ranges, hist, status, tgt[3], log, logcount,
         bigq,       // per-primitive first pair index
         clipq,      // triangles queued for the clipper
@@ -411,9 +411,11 @@ void collect_stats(swr_context *c)
 
 // Device memory one triangle draw works in, beyond its inputs and render targets.
 struct Arenas {
-    uint2 *app = nullptr, *app_ex = nullptr;
+    uint32_t *cnt = nullptr;
+    uint8_t *cflag = nullptr;
+    uint2 *app = nullptr, *ex = nullptr;
+    uint4 *app_ex = nullptr;
     uint32_t *live = nullptr, *clipq = nullptr, *clipq_cnt = nullptr;
-    uint2 *grp = nullptr, *grp_ex = nullptr;
     void *scan_tmp = nullptr;
     uint32_t *ranges = nullptr;
     float *prims = nullptr;
@@ -426,19 +428,22 @@ struct Arenas {
 
 // Sizes of the arenas that depend only on the input (triangles, batches, tiles).
 struct FixedSizes {
-    size_t app, live, clipq, clipq_cnt, grp, scan_tmp, ranges;
+    size_t cnt, cflag, ex, app, app_ex, live, clipq, clipq_cnt, scan_tmp, ranges;
 };
 
-FixedSizes fixed_sizes(size_t T, uint64_t ngrp, uint32_t tiles)
+FixedSizes fixed_sizes(size_t T, uint64_t batches, uint32_t tiles)
 {
     FixedSizes f;
-    f.app = T * 8;
+    f.cnt = batches * BATCH * 4;
+    f.cflag = batches * BATCH;
+    f.ex = batches * BATCH * 8;
+    f.app = batches * BATCH * 8;
+    f.app_ex = T * 16;
     f.live = T * 4;
     const size_t blocks = (T + 255) / 256, per_region = ((blocks + 63) / 64) * 256;
     f.clipq = 64 * per_region * 4;
     f.clipq_cnt = DRAW_COUNTER_WORDS * 4;
-    f.grp = ngrp * 8;
-    f.scan_tmp = (scan_tmp_elems(T) + scan_tmp_elems(ngrp)) * 8;
+    f.scan_tmp = fan_scan_bytes(batches);
     f.ranges = (size_t)tiles * 8;
     return f;
 }
@@ -504,30 +509,30 @@ void *scratch_of(int device)
 // Lays every arena of a draw out in [base, base + bytes): the input-sized ones first, then
 // primitive records and tile pairs from what remains.  Returns false when the input-sized
 // arenas and a minimal record / pair capacity do not fit.
-bool carve_arenas(unsigned char *base, size_t bytes, size_t T, uint64_t ngrp, uint32_t tiles,
+bool carve_arenas(unsigned char *base, size_t bytes, size_t T, uint64_t batches, uint32_t tiles,
                   int stride_words, Arenas &A)
 {
-    const FixedSizes f = fixed_sizes(T, ngrp, tiles);
+    const FixedSizes f = fixed_sizes(T, batches, tiles);
     size_t off = 0;
     auto take = [&](size_t n) -> unsigned char * {
         unsigned char *p = base + off;
         off += (std::max<size_t>(n, 1) + 255) & ~(size_t)255;
         return p;
     };
-    const size_t fixed_total = 2 * ((f.app + 255) & ~(size_t)255) + ((f.live + 255) & ~(size_t)255) +
-                               ((f.clipq + 255) & ~(size_t)255) +
-                               ((f.clipq_cnt + 255) & ~(size_t)255) +
-                               2 * ((f.grp + 255) & ~(size_t)255) +
-                               ((f.scan_tmp + 255) & ~(size_t)255) + ((f.ranges + 255) & ~(size_t)255);
+    size_t fixed_total = 0;
+    for (size_t n : {f.cnt, f.cflag, f.ex, f.app, f.app_ex, f.live, f.clipq, f.clipq_cnt,
+                     f.scan_tmp, f.ranges})
+        fixed_total += (n + 255) & ~(size_t)255;
     if (fixed_total >= bytes)
         return false;
+    A.cnt = (uint32_t *)take(f.cnt);
+    A.cflag = (uint8_t *)take(f.cflag);
+    A.ex = (uint2 *)take(f.ex);
     A.app = (uint2 *)take(f.app);
-    A.app_ex = (uint2 *)take(f.app);
+    A.app_ex = (uint4 *)take(f.app_ex);
     A.live = (uint32_t *)take(f.live);
     A.clipq = (uint32_t *)take(f.clipq);
     A.clipq_cnt = (uint32_t *)take(f.clipq_cnt);
-    A.grp = (uint2 *)take(f.grp);
-    A.grp_ex = (uint2 *)take(f.grp);
     A.scan_tmp = take(f.scan_tmp);
     A.ranges = (uint32_t *)take(f.ranges);
     // records: every input triangle and an eighth more for clip fans; pairs: the rest
@@ -651,35 +656,36 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
     }
 
     const uint32_t batches = (uint32_t)((T + BATCH - 1) / BATCH);
-    const uint64_t ngrp = (uint64_t)batches * 2048;
     Arenas A;
     if (noalloc) {
         unsigned char *base = static_cast<unsigned char *>(scratch_of(c->device));
         if (!base)
             return fail(c, SWR_ERR_HIP, "the device address of the scratch array is unknown");
-        if (!carve_arenas(base, SWR_NOALLOC_SCRATCH_BYTES, T, ngrp, tiles, L.stride, A))
+        if (!carve_arenas(base, SWR_NOALLOC_SCRATCH_BYTES, T, batches, tiles, L.stride, A))
             return fail(c, SWR_ERR_CAPACITY,
                         "%zu triangles on %u tiles do not fit the %d-byte scratch array of "
                         "swr_draw_elements_noalloc",
                         T, tiles, SWR_NOALLOC_SCRATCH_BYTES);
     } else {
-        const FixedSizes f = fixed_sizes(T, ngrp, tiles);
+        const FixedSizes f = fixed_sizes(T, batches, tiles);
         HIP_TRY(c, ensure(c, c->app, f.app));
         HIP_TRY(c, ensure(c, c->clipq, f.clipq));
         HIP_TRY(c, ensure(c, c->clipq_cnt, f.clipq_cnt));
-        HIP_TRY(c, ensure(c, c->app_ex, f.app));
+        HIP_TRY(c, ensure(c, c->app_ex, f.app_ex));
         HIP_TRY(c, ensure(c, c->live, f.live));
-        HIP_TRY(c, ensure(c, c->grp, f.grp));
-        HIP_TRY(c, ensure(c, c->grp_ex, f.grp));
+        HIP_TRY(c, ensure(c, c->cnt, f.cnt));
+        HIP_TRY(c, ensure(c, c->cflag, f.cflag));
+        HIP_TRY(c, ensure(c, c->ex, f.ex));
         HIP_TRY(c, ensure(c, c->scan_tmp, f.scan_tmp));
         HIP_TRY(c, ensure(c, c->ranges, f.ranges));
         A.app = (uint2 *)c->app.p;
-        A.app_ex = (uint2 *)c->app_ex.p;
+        A.app_ex = (uint4 *)c->app_ex.p;
         A.live = (uint32_t *)c->live.p;
         A.clipq = (uint32_t *)c->clipq.p;
         A.clipq_cnt = (uint32_t *)c->clipq_cnt.p;
-        A.grp = (uint2 *)c->grp.p;
-        A.grp_ex = (uint2 *)c->grp_ex.p;
+        A.cnt = (uint32_t *)c->cnt.p;
+        A.cflag = (uint8_t *)c->cflag.p;
+        A.ex = (uint2 *)c->ex.p;
         A.scan_tmp = c->scan_tmp.p;
         A.ranges = (uint32_t *)c->ranges.p;
         c->prim_cap = std::max<uint64_t>(c->prim_cap, T + 256);
@@ -767,8 +773,9 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
         g.app = A.app;
         g.app_ex = A.app_ex;
         g.live = window_input ? nullptr : A.live;
-        g.grp = A.grp;
-        g.grp_ex = A.grp_ex;
+        g.cnt = A.cnt;
+        g.cflag = A.cflag;
+        g.ex = A.ex;
         g.prims = A.prims;
         g.prim_cap = A.prim_cap;
         g.pair_keys = A.pk_a;
@@ -797,13 +804,8 @@ int draw_triangles(swr_context *c, const int32_t *indices, size_t count, bool wi
         HIP_TRY(c, launch_begin(g, c->stream));
         HIP_TRY(c, launch_geom_count(g, c->stream));
         record(c, 1);
-        if (!window_input)
-            HIP_TRY(c, scan_fans_and_pairs(g.app, A.app_ex, T, A.live, g.grp, A.grp_ex, ngrp,
-                                           A.scan_tmp, g.status, A.prim_cap, A.pair_cap,
-                                           c->stream));
-        else
-            HIP_TRY(c, scan_pairs(g.grp, A.grp_ex, ngrp, (uint2 *)A.scan_tmp, g.status,
-                                  A.prim_cap, A.pair_cap, c->stream));
+        HIP_TRY(c, scan_fans(A.cnt, A.cflag, A.app, A.ex, A.app_ex, g.live, batches, A.scan_tmp,
+                             g.status, A.prim_cap, A.pair_cap, c->stream));
         record(c, 2);
         HIP_TRY(c, launch_geom_emit(g, c->stream));
         HIP_TRY(c, launch_expand(g, c->stream, expand_chunk_of(c->tune.expand_chunk, A.pair_cap)));
@@ -1246,9 +1248,8 @@ int swr_destroy(swr_context *c)
         return SWR_ERR_INVALID_ARG;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    DevBuf *bufs[] = {&c->idx, &c->attr0, &c->wverts, &c->app, &c->app_ex, &c->live, &c->grp,
-                      &c->grp_ex,
-                      &c->scan_tmp, &c->prims, &c->pk_a, &c->pv_a, &c->pk_b, &c->pv_b,
+    DevBuf *bufs[] = {&c->idx, &c->attr0, &c->wverts, &c->app, &c->app_ex, &c->live, &c->cnt,
+                      &c->cflag, &c->ex, &c->scan_tmp, &c->prims, &c->pk_a, &c->pv_a, &c->pk_b, &c->pv_b,
                       &c->ranges, &c->hist, &c->status, &c->tgt[0],
                       &c->tgt[1], &c->tgt[2], &c->log, &c->logcount, &c->bigq, &c->clipq,
                       &c->clipq_cnt, &c->chunk_kept, &c->vwin, &c->vmask, &c->vmod_out,

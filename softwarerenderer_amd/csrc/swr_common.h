@@ -241,6 +241,10 @@ struct SceneDev {
     uint32_t tris, batch0;
 };
 
+// Flags of an input triangle's counts: the main pass emits it (not the clip queue); clipping
+// appended fan triangles to its batch.
+constexpr uint32_t COUNT_LIVE = 1u, COUNT_APPENDS = 2u;
+
 // ---- launch arguments ---------------------------------------------------------------
 struct GeomArgs {
     // input
@@ -266,11 +270,16 @@ struct GeomArgs {
     const swr_rasterizer_vertex *wverts;
     uint64_t wvert_count;
     // scan buffers
-    uint2 *app;                 // [tris] (fan triangles appended, live) per input triangle
-    const uint2 *app_ex;        // exclusive scan of app
+    uint32_t *cnt;              // [batches*1024] pairs of each input triangle's first fan
+                                // triangle, 0 when it draws nothing
+    uint8_t *cflag;             // [batches*1024] COUNT_LIVE, COUNT_APPENDS
+    uint2 *app;                 // [batches*1024] {fan triangles appended | drawn ones << 16, their
+                                // pairs}, valid where COUNT_APPENDS is set
+    const uint2 *ex;            // [batches*1024] (primitives, pairs) before the first fan
+                                // triangle, valid where cnt is not 0
+    const uint4 *app_ex;        // [tris] {primitives, pairs before the appended ones, fans the
+                                // batch has appended before}, valid where COUNT_APPENDS is set
     uint32_t *live;             // [tris] the live triangles in order (nullptr: emit walks all)
-    uint2 *grp;                 // [batches*2048] (prims, pairs) per (batch, phase, j)
-    const uint2 *grp_ex;        // exclusive scan of grp
     // outputs
     float *prims;               // records
     uint64_t prim_cap;

@@ -753,8 +753,8 @@ __device__ inline void interp_pixel(const DiffArgs &d, const PixelIdx &pi, bool 
         bool pf;
         int cur;
         walk[dir] = qx < d.W && qy < d.H && pair_start(d, view, px, py, qx, qy, pf, cur);
-        d.pflag[2 * i + dir] = 0;
     }
+    reinterpret_cast<uint16_t *>(d.pflag)[i] = 0;
 }
 
 template <int C>

@@ -768,9 +768,9 @@ __device__ __forceinline__ int clip_one_plane(const GeomArgs &a, const Pos4 *P,
 // LISTED: the emit pass over the compacted list of triangles the count pass found live (a
 // workgroup's triangles may then come from several batches and scenes).
 //
-// The count pass writes app[t] = (fan triangles appended, live): live when the main pass
-// itself emits a primitive for t (a triangle the clip queue takes is not live).  Their scan
-// gives the appended fans' draw-order slots and, with the live flags, the compacted list.
+// The count pass writes t's counts and flags: live when the main pass itself emits a primitive
+// for t (a triangle the clip queue takes is not live).  Their scan gives the primitives' places
+// in draw order and, with the live flags, the compacted list.
 template <int NV, bool EMIT, bool LISTED = false>
 __device__ void process_triangle(const GeomArgs &a0, uint32_t t, uint32_t usid = 0)
 {
@@ -806,21 +806,15 @@ __device__ void process_triangle(const GeomArgs &a0, uint32_t t, uint32_t usid =
     const uint32_t nbt = (c.kb + 1 < nbatches) ? (uint32_t)BATCH : ntris - c.kb * (uint32_t)BATCH;
     if (!live) {
         if (!EMIT) {
-            a.app[t] = make_uint2(0, 0);
-            a.grp[(size_t)c.b * 2048 + c.j] = make_uint2(0, 0);
-            a.grp[(size_t)c.b * 2048 + 1024 + c.j] = make_uint2(0, 0);
+            a.cnt[t] = 0;
+            a.cflag[t] = 0;
         }
         return;
     }
     if (EMIT) {
-        if (!a.window_input)
-            c.slot1 = nbt + (a.app_ex[t].x - a.app_ex[c.b * BATCH].x);
-        uint2 g0 = a.grp_ex[(size_t)c.b * 2048 + c.j];
-        uint2 g1 = a.grp_ex[(size_t)c.b * 2048 + 1024 + c.j];
+        const uint2 g0 = a.ex[t];
         c.pos0 = g0.x;
         c.pairs0 = g0.y;
-        c.pos1 = g1.x;
-        c.pairs1 = g1.y;
     }
     constexpr int NVS = NV > 0 ? NV : 1;
     float var3[3][NVS];
@@ -911,6 +905,12 @@ __device__ void process_triangle(const GeomArgs &a0, uint32_t t, uint32_t usid =
             } else if (fully_clipped_early(P, cm)) {
                 nfan = 0;
             } else if (one_plane_case(P, cm, dp1)) {
+                if (EMIT) {  // read where clipping appends a fan triangle
+                    const uint4 g1 = a.app_ex[t];
+                    c.pos1 = g1.x;
+                    c.pairs1 = g1.y;
+                    c.slot1 = nbt + g1.z;
+                }
                 nfan = clip_one_plane<NVS, EMIT>(a, P, var3, dp1, W, V);
             } else {
                 if (!EMIT) {  // the queue kernels clip it and write its counts
@@ -939,10 +939,11 @@ fans:
         fan_triangle<NV, EMIT>(a, c, k, W[0], wb, wc, V[0], vb, vc, cull);
     }
     if (!EMIT) {
-        a.grp[(size_t)c.b * 2048 + c.j] = make_uint2(c.cnt0, c.cntp0);
-        a.grp[(size_t)c.b * 2048 + 1024 + c.j] = make_uint2(c.cnt1, c.cntp1);
-        if (!a.window_input)
-            a.app[t] = make_uint2(c.app_n, c.cnt0 + c.cnt1 > 0 ? 1u : 0u);
+        a.cnt[t] = c.cntp0;
+        a.cflag[t] = (uint8_t)((c.cnt0 + c.cnt1 > 0 ? COUNT_LIVE : 0u) |
+                               (c.app_n ? COUNT_APPENDS : 0u));
+        if (c.app_n)
+            a.app[t] = make_uint2(c.app_n | c.cnt1 << 16, c.cntp1);
     }
 }
 
@@ -975,13 +976,11 @@ __global__ void __launch_bounds__(256) k_begin(GeomArgs a)
     if (a.vwin)
         for (uint32_t v = i; v < a.nverts; v += gridDim.x * blockDim.x)
             shade_vertex(a, v);
-    // the last batch's unused (batch, phase, j) slots count nothing
+    // the last batch's unused places count nothing
     uint32_t tail = a.batches * 1024u - a.tris;
     for (uint32_t k = i; k < tail; k += gridDim.x * blockDim.x) {
-        uint32_t tt = a.tris + k;
-        uint32_t bb = tt >> 10, jj = tt & 1023u;
-        a.grp[(size_t)bb * 2048 + jj] = make_uint2(0, 0);
-        a.grp[(size_t)bb * 2048 + 1024 + jj] = make_uint2(0, 0);
+        a.cnt[a.tris + k] = 0;
+        a.cflag[a.tris + k] = 0;
     }
 }
 
@@ -1082,7 +1081,7 @@ __device__ inline WinV shfl_win(const WinV &w, int src)
 }
 
 // One queued triangle t, clipped by the calling wave (all 64 lanes, t uniform).  The count
-// pass writes its (batch, phase, j) counts and appended-fan count; the emit pass its records.
+// pass writes its counts; the emit pass its records.
 template <int NV, bool EMIT>
 __device__ void clip_queued(const GeomArgs &a0, uint32_t t, ClipStage<NV> &st)
 {
@@ -1106,13 +1105,13 @@ __device__ void clip_queued(const GeomArgs &a0, uint32_t t, ClipStage<NV> &st)
     uint64_t pos0 = 0, pairs0 = 0, pos1 = 0, pairs1 = 0;
     if (EMIT) {
         const uint32_t nbt = (kb + 1 < nbatches) ? (uint32_t)BATCH : ntris - kb * (uint32_t)BATCH;
-        slot1 = nbt + (a.app_ex[t].x - a.app_ex[b * BATCH].x);
-        const uint2 g0 = a.grp_ex[(size_t)b * 2048 + j];
-        const uint2 g1 = a.grp_ex[(size_t)b * 2048 + 1024 + j];
+        const uint2 g0 = a.ex[t];
         pos0 = g0.x;
         pairs0 = g0.y;
+        const uint4 g1 = a.app_ex[t];  // used where clipping appends fan triangles
         pos1 = g1.x;
         pairs1 = g1.y;
+        slot1 = nbt + g1.z;
     }
     // lanes 0-2: the input vertices
     Pos4 P = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1219,10 +1218,11 @@ __device__ void clip_queued(const GeomArgs &a0, uint32_t t, ClipStage<NV> &st)
     if (!EMIT) {
         const uint32_t tot1 = __shfl(incl, 63);
         if (lane == 0) {
-            a.grp[(size_t)b * 2048 + j] = make_uint2(drawn ? 1u : 0u, nt);
-            a.grp[(size_t)b * 2048 + 1024 + j] =
-                make_uint2((uint32_t)__popcll(m_drawn & ~1ull), tot1);
-            a.app[t] = make_uint2(n > 3 ? (uint32_t)(n - 3) : 0u, 0u);
+            a.cnt[t] = nt;
+            a.cflag[t] = n > 3 ? COUNT_APPENDS : 0u;
+            if (n > 3)
+                a.app[t] = make_uint2(
+                    (uint32_t)(n - 3) | (uint32_t)__popcll(m_drawn & ~1ull) << 16, tot1);
         }
         return;
     }
@@ -1238,8 +1238,8 @@ __device__ void clip_queued(const GeomArgs &a0, uint32_t t, ClipStage<NV> &st)
     fan_write<NV>(a, pos, pb, nt, key, src, sid, g, w0, w1, w2, v0, v1, v2, swap);
 }
 
-// The queued triangles, densely packed (order does not matter: each writes its own (batch,
-// phase, j) counts and draw-order positions).  Wave `wid` of `nwaves` prefix-sums the region
+// The queued triangles, densely packed (order does not matter: each writes its own
+// counts and draw-order positions).  Wave `wid` of `nwaves` prefix-sums the region
 // counts into its own s_off, then takes dense indices wid, wid + nwaves, ... and maps each
 // to its (region, slot); s_off and st are the wave's own LDS.
 template <int NV, bool EMIT>

@@ -53,16 +53,15 @@ uint64_t scan_tmp_elems(uint64_t n);
 hipError_t scan_lines(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
                       const unsigned long long *parts, uint32_t nparts,
                       unsigned long long *status, hipStream_t s);
-hipError_t scan_pairs(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
-                      unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
-                      hipStream_t s);
-// the (appended fans, live) scan of the input triangles, compacting the live ones into
-// `live`, and scan_pairs of the slot counts, in shared launches; tmp holds
-// scan_tmp_elems(na) + scan_tmp_elems(ng) 8-byte elements
-hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uint32_t *live,
-                               const uint2 *grp, uint2 *grp_ex, uint64_t ng, void *tmp,
-                               unsigned long long *status, uint64_t cap_prims,
-                               uint64_t cap_pairs, hipStream_t s);
+// The draw-order places of a draw's primitives and pairs: per batch of 1024 input triangles,
+// first every triangle's first fan triangle, then the appended ones.  Takes the counts (cnt,
+// cflag, app as GeomArgs states them), writes ex and app_ex, compacts the live triangles into
+// `live` (may be null) and publishes the totals.  tmp holds fan_scan_bytes(batches).
+size_t fan_scan_bytes(uint64_t batches);
+hipError_t scan_fans(const uint32_t *cnt, const uint8_t *cflag, const uint2 *app, uint2 *ex,
+                     uint4 *app_ex, uint32_t *live, uint64_t batches, void *tmp,
+                     unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
+                     hipStream_t s);
 hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tiles, hipStream_t s);
 hipError_t launch_ranges(const SortBuffers &sb, unsigned long long *status, uint32_t tiles,
                          hipStream_t s);

@@ -27,25 +27,41 @@ constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
 __device__ inline uint32_t sadd(uint32_t a, uint32_t b) { return a + b; }
 __device__ inline uint2 sadd(uint2 a, uint2 b) { return make_uint2(a.x + b.x, a.y + b.y); }
+__device__ inline uint4 sadd(uint4 a, uint4 b)
+{
+    return make_uint4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
 template <typename T> __device__ inline T szero();
 template <> __device__ inline uint32_t szero<uint32_t>() { return 0u; }
 template <> __device__ inline uint2 szero<uint2>() { return make_uint2(0u, 0u); }
+template <> __device__ inline uint4 szero<uint4>() { return make_uint4(0u, 0u, 0u, 0u); }
 
-// Wave-wide inclusive scan (64 lanes, shuffles).
+// Wave-wide inclusive scan of 64 lanes: DPP steps inside the rows of 16 lanes, then the rows'
+// totals handed on (a shuffle per step waits for the LDS six times over).
 __device__ inline uint32_t wave_incl(uint32_t v)
 {
-    const int lane = (int)(threadIdx.x & 63u);
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t o = __shfl_up(v, off, 64);
-        if (lane >= off)
-            v += o;
-    }
+#define SWR_SCAN_STEP(CTRL, ROWS) \
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false)
+    SWR_SCAN_STEP(0x111, 0xF);  // row_shr 1, 2, 4, 8
+    SWR_SCAN_STEP(0x112, 0xF);
+    SWR_SCAN_STEP(0x114, 0xF);
+    SWR_SCAN_STEP(0x118, 0xF);
+    SWR_SCAN_STEP(0x142, 0xA);  // row_bcast 15, 31
+    SWR_SCAN_STEP(0x143, 0xC);
+#undef SWR_SCAN_STEP
     return v;
 }
 __device__ inline uint2 wave_incl(uint2 v) { return make_uint2(wave_incl(v.x), wave_incl(v.y)); }
+__device__ inline uint4 wave_incl(uint4 v)
+{
+    return make_uint4(wave_incl(v.x), wave_incl(v.y), wave_incl(v.z), wave_incl(v.w));
+}
 __device__ inline uint32_t ssub(uint32_t a, uint32_t b) { return a - b; }
 __device__ inline uint2 ssub(uint2 a, uint2 b) { return make_uint2(a.x - b.x, a.y - b.y); }
+__device__ inline uint4 ssub(uint4 a, uint4 b)
+{
+    return make_uint4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w);
+}
 
 // Block-wide exclusive scan of one value per thread; returns the block total in *total.
 template <typename T>
@@ -188,14 +204,11 @@ __device__ T block_carry(const T *sums, uint32_t b)
 
 // Writes the exclusive scan.  CARRY: the block adds up the block sums before it (the
 // two-kernel scan); else sums[] holds their exclusive scan.  With `status` set the thread
-// that owns the last element publishes the total (publish_totals).  With `list` (the
-// (appended fans, live) scan of the geometry pass): element i with a live flag writes i at
-// position (its exclusive live count), compacting the live triangles in order, and the
-// live total goes to status[ST_LIVE].
+// that owns the last element publishes the total (publish_totals).
 template <typename T, bool CARRY>
 __device__ void down_tile(const T *in, uint64_t n, const T *sums, T *out,
                           unsigned long long *status, uint64_t cap_x, uint64_t cap_y,
-                          uint32_t b, uint32_t *list = nullptr)
+                          uint32_t b)
 {
     const T carry = CARRY ? block_carry<T>(sums, b) : sums[b];
     const uint64_t base = (uint64_t)b * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
@@ -211,15 +224,7 @@ __device__ void down_tile(const T *in, uint64_t n, const T *sums, T *out,
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         o[i] = run;
-        if constexpr (sizeof(T) == 8) {
-            if (list) {
-                if (base + i < n && vals[i].y)
-                    list[run.y] = (uint32_t)(base + i);
-                if (base + i == n - 1)
-                    status[ST_LIVE] = run.y + vals[i].y;
-            }
-        }
-        if (status && !list && base + i == n - 1)
+        if (status && base + i == n - 1)
             publish_totals(sadd(run, vals[i]), status, cap_x, cap_y);
         run = sadd(run, vals[i]);
     }
@@ -230,34 +235,9 @@ template <typename T, bool CARRY>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_down(const T *in, uint64_t n,
                                                           const T *sums, T *out,
                                                           unsigned long long *status,
-                                                          uint64_t cap_x, uint64_t cap_y,
-                                                          uint32_t *list)
+                                                          uint64_t cap_x, uint64_t cap_y)
 {
-    down_tile<T, CARRY>(in, n, sums, out, status, cap_x, cap_y, blockIdx.x, list);
-}
-
-// The per-triangle (appended fans, live) counts and the per-slot (primitives, pairs) counts
-// scanned together: blocks [0, nb_a) take the first, the rest the second.
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_reduce2(const uint2 *a, uint64_t na,
-                                                             uint2 *sa, uint32_t nba,
-                                                             const uint2 *g, uint64_t ng,
-                                                             uint2 *sg)
-{
-    if (blockIdx.x < nba)
-        reduce_tile<uint2>(a, na, sa, blockIdx.x);
-    else
-        reduce_tile<uint2>(g, ng, sg, blockIdx.x - nba);
-}
-
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_down2(
-    const uint2 *a, uint64_t na, const uint2 *sa, uint2 *oa, uint32_t nba, uint32_t *list,
-    const uint2 *g, uint64_t ng, const uint2 *sg, uint2 *og, unsigned long long *status,
-    uint64_t cap_x, uint64_t cap_y)
-{
-    if (blockIdx.x < nba)
-        down_tile<uint2, true>(a, na, sa, oa, status, 0, 0, blockIdx.x, list);
-    else
-        down_tile<uint2, true>(g, ng, sg, og, status, cap_x, cap_y, blockIdx.x - nba);
+    down_tile<T, CARRY>(in, n, sums, out, status, cap_x, cap_y, blockIdx.x);
 }
 
 // Scans of up to this many blocks skip the pass over the block sums: each block of the
@@ -267,8 +247,7 @@ constexpr uint32_t SCAN_CARRY_BLOCKS = 8192;
 
 template <typename T>
 hipError_t scan_impl(const T *in, T *out, uint64_t n, T *tmp, unsigned long long *status,
-                     uint64_t cap_x, uint64_t cap_y, hipStream_t s,
-                     uint32_t *list = nullptr)
+                     uint64_t cap_x, uint64_t cap_y, hipStream_t s)
 {
     if (!n)
         return hipSuccess;
@@ -276,11 +255,11 @@ hipError_t scan_impl(const T *in, T *out, uint64_t n, T *tmp, unsigned long long
     hipLaunchKernelGGL(k_scan_reduce<T>, dim3(nb), dim3(SCAN_THREADS), 0, s, in, n, tmp);
     if (nb <= SCAN_CARRY_BLOCKS) {
         hipLaunchKernelGGL((k_scan_down<T, true>), dim3(nb), dim3(SCAN_THREADS), 0, s, in, n,
-                           tmp, out, status, cap_x, cap_y, list);
+                           tmp, out, status, cap_x, cap_y);
     } else {
         hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nb);
         hipLaunchKernelGGL((k_scan_down<T, false>), dim3(nb), dim3(SCAN_THREADS), 0, s, in, n,
-                           tmp, out, status, cap_x, cap_y, list);
+                           tmp, out, status, cap_x, cap_y);
     }
     return hipGetLastError();
 }
@@ -320,33 +299,284 @@ hipError_t scan_lines(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
     return hipGetLastError();
 }
 
-hipError_t scan_pairs(const uint2 *in, uint2 *out, uint64_t n, uint2 *tmp,
-                      unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
-                      hipStream_t s)
+// ---- the draw-order places of a draw's primitives -------------------------------------------
+// A wave takes a batch of 1024 input triangles, a workgroup FAN_BATCHES batches.  Bound by the
+// bytes: a triangle's counts are 5 bytes here (a word of pairs and a byte of flags), 8 bytes of
+// places are written where it draws, and the appended fans' counts are read only where clipping
+// made some.  As one element per triangle for the live list and two per triangle for the
+// places, 8 bytes each, read twice and written once, the scans of 5.2M triangles (64 views of
+// 82k) took 80 us and now take 18; of 1M, 30% of them clipped, 21 and now 11 us; with few
+// workgroups both are a chain of loads and scans (150k triangles: 10 us both ways).
+constexpr uint32_t FAN_BATCHES = SCAN_THREADS / 64;
+static_assert(BATCH == 1024, "16 triangles per lane");
+static_assert(BATCH * (MAX_CLIP - 3) < 65536, "a batch's appended fans count in 16 bits");
+
+// The lane's 16 triangles of batch b: words w and flag bytes f of triangles
+// 256 r + 4 lane .. + 3 for r = 0 .. 3.
+__device__ inline void fan_load(const uint32_t *cnt, const uint8_t *cflag, uint32_t b,
+                                uint32_t lane, uint4 (&w)[4], uint32_t (&f)[4])
 {
-    return scan_impl<uint2>(in, out, n, tmp, status, cap_prims, cap_pairs, s);
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+        w[r] = reinterpret_cast<const uint4 *>(cnt)[(size_t)b * 256 + r * 64 + lane];
+        f[r] = reinterpret_cast<const uint32_t *>(cflag)[(size_t)b * 256 + r * 64 + lane];
+    }
 }
 
-hipError_t scan_fans_and_pairs(const uint2 *app, uint2 *app_ex, uint64_t na, uint32_t *live,
-                               const uint2 *grp, uint2 *grp_ex, uint64_t ng, void *tmp,
-                               unsigned long long *status, uint64_t cap_prims,
-                               uint64_t cap_pairs, hipStream_t s)
+__device__ inline uint32_t item(const uint4 &w, int i)
 {
-    const uint32_t nba = (uint32_t)((na + SCAN_TILE - 1) / SCAN_TILE);
-    const uint32_t nbg = (uint32_t)((ng + SCAN_TILE - 1) / SCAN_TILE);
-    // block sums: those of the first scan, then those of the second
-    uint2 *sa = static_cast<uint2 *>(tmp);
-    uint2 *sg = sa + scan_tmp_elems(na);
-    if (!na || !ng || nba > SCAN_CARRY_BLOCKS || nbg > SCAN_CARRY_BLOCKS) {
-        hipError_t e = scan_impl<uint2>(app, app_ex, na, sa, status, 0, 0, s, live);
-        if (e != hipSuccess)
-            return e;
-        return scan_pairs(grp, grp_ex, ng, sg, status, cap_prims, cap_pairs, s);
+    return i == 0 ? w.x : (i == 1 ? w.y : (i == 2 ? w.z : w.w));
+}
+
+// The appended counts of the same triangles, two to a uint4; the loads leave together.
+__device__ inline void fan_load_appended(const uint2 *app, uint32_t b, uint32_t lane,
+                                         uint4 (&q)[4][2])
+{
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            q[r][k] = reinterpret_cast<const uint4 *>(
+                app + (size_t)b * BATCH + r * 256 + 4 * lane)[k];
+}
+
+// Triangle i's appended counts, 0 where there are none.
+__device__ inline uint2 appended(const uint4 (&q)[2], uint32_t f, int i)
+{
+    const bool has = (f >> (8 * i)) & COUNT_APPENDS;
+    const uint4 &h = q[i >> 1];
+    return make_uint2(has ? (i & 1 ? h.z : h.x) : 0u, has ? (i & 1 ? h.w : h.y) : 0u);
+}
+
+__device__ inline bool fan_appends(const uint32_t (&f)[4])
+{
+    return __ballot((f[0] | f[1] | f[2] | f[3]) & (COUNT_APPENDS * 0x01010101u)) != 0ull;
+}
+
+// {primitives, pairs, live} of the lane's triangles, appended ones (any) included.
+__device__ inline uint4 fan_sum(const uint4 (&w)[4], const uint32_t (&f)[4], bool any,
+                                const uint4 (&q)[4][2])
+{
+    uint4 t = szero<uint4>();
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t c = item(w[r], i);
+            t.x += c ? 1u : 0u;
+            t.y += c;
+            t.z += (f[r] >> (8 * i)) & COUNT_LIVE ? 1u : 0u;
+        }
+    if (any) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint2 x = appended(q[r], f[r], i);
+                t.x += x.x >> 16;
+                t.y += x.y;
+            }
     }
-    hipLaunchKernelGGL(k_scan_reduce2, dim3(nba + nbg), dim3(SCAN_THREADS), 0, s, app, na, sa,
-                       nba, grp, ng, sg);
-    hipLaunchKernelGGL(k_scan_down2, dim3(nba + nbg), dim3(SCAN_THREADS), 0, s, app, na, sa,
-                       app_ex, nba, live, grp, ng, sg, grp_ex, status, cap_prims, cap_pairs);
+    return t;
+}
+
+// The lane's share of batch b's sum.
+__device__ inline uint4 batch_sum(const uint32_t *cnt, const uint8_t *cflag, const uint2 *app,
+                                  uint32_t b, uint32_t lane)
+{
+    uint4 w[4], q[4][2];
+    uint32_t f[4];
+    fan_load(cnt, cflag, b, lane, w, f);
+    const bool any = fan_appends(f);
+    if (any)
+        fan_load_appended(app, b, lane, q);
+    return fan_sum(w, f, any, q);
+}
+
+__device__ inline uint32_t wave_sum(uint32_t v)
+{
+    return __builtin_amdgcn_readlane(wave_incl(v), 63);
+}
+__device__ inline uint4 wave_sum(uint4 v)
+{
+    return make_uint4(wave_sum(v.x), wave_sum(v.y), wave_sum(v.z), 0u);
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_fan_reduce(const uint32_t *cnt,
+                                                           const uint8_t *cflag,
+                                                           const uint2 *app, uint32_t batches,
+                                                           uint4 *sums)
+{
+    __shared__ uint4 s_w[FAN_BATCHES];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t b = blockIdx.x * FAN_BATCHES + wv;
+    uint4 t = wave_sum(b < batches ? batch_sum(cnt, cflag, app, b, lane) : szero<uint4>());
+    if (lane == 0)
+        s_w[wv] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t k = 1; k < FAN_BATCHES; ++k)
+            t = sadd(t, s_w[k]);
+        sums[blockIdx.x] = t;
+    }
+}
+
+// CARRY: what lies before the workgroup is FAN_COUNTS: added up here from the counts
+// themselves, FAN_SUMS: from the workgroups' sums, FAN_SCANNED: already scanned.
+constexpr int FAN_COUNTS = 0, FAN_SUMS = 1, FAN_SCANNED = 2;
+
+template <int CARRY>
+__global__ void __launch_bounds__(SCAN_THREADS) k_fan_down(
+    const uint32_t *cnt, const uint8_t *cflag, const uint2 *app, uint32_t batches,
+    const uint4 *sums, uint2 *ex, uint4 *app_ex, uint32_t *live, unsigned long long *status,
+    uint64_t cap_prims, uint64_t cap_pairs)
+{
+    __shared__ uint4 s_own[FAN_BATCHES], s_carry[FAN_BATCHES];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t b = blockIdx.x * FAN_BATCHES + wv;
+    uint4 w[4];
+    uint32_t f[4];
+    uint4 carry = szero<uint4>(), own = szero<uint4>();
+    uint4 xq[4][2];
+    bool any = false;
+    const bool mine = b < batches;
+    if (mine) {
+        fan_load(cnt, cflag, b, lane, w, f);
+        any = fan_appends(f);
+        if (any)
+            fan_load_appended(app, b, lane, xq);
+        own = fan_sum(w, f, any, xq);
+    }
+    if (CARRY == FAN_COUNTS) {
+        for (uint32_t k = wv; k < blockIdx.x * FAN_BATCHES; k += FAN_BATCHES)
+            carry = sadd(carry, batch_sum(cnt, cflag, app, k, lane));
+    } else if (CARRY == FAN_SUMS) {
+        for (uint32_t k = threadIdx.x; k < blockIdx.x; k += SCAN_THREADS)
+            carry = sadd(carry, sums[k]);
+    } else if (threadIdx.x == 0) {
+        carry = sums[blockIdx.x];
+    }
+    carry = wave_sum(carry);
+    own = wave_sum(own);
+    if (lane == 0) {
+        s_carry[wv] = carry;
+        s_own[wv] = own;
+    }
+    __syncthreads();
+    if (!mine)
+        return;
+    uint4 run = szero<uint4>();
+#pragma unroll
+    for (uint32_t k = 0; k < FAN_BATCHES; ++k) {
+        run = sadd(run, s_carry[k]);
+        if (k < wv)
+            run = sadd(run, s_own[k]);
+    }
+    if (b + 1 == batches && lane == 0) {
+        const uint4 t = sadd(run, own);
+        publish_totals(make_uint2(t.x, t.y), status, cap_prims, cap_pairs);
+        if (live)
+            status[ST_LIVE] = t.z;
+    }
+    // the first fan triangles and the live list
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+        const uint32_t t0 = b * (uint32_t)BATCH + r * 256 + 4 * lane;
+        uint2 s = make_uint2(0u, 0u);  // {primitives | live << 16, pairs}
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t c = item(w[r], i), g = f[r] >> (8 * i);
+            s.x += (c ? 1u : 0u) | (g & COUNT_LIVE ? 0x10000u : 0u);
+            s.y += c;
+        }
+        const uint2 inc = wave_incl(s);
+        uint32_t p = run.x + ((inc.x - s.x) & 0xFFFFu), q = run.y + (inc.y - s.y),
+                 l = run.z + ((inc.x - s.x) >> 16);
+        uint2 o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t c = item(w[r], i), g = f[r] >> (8 * i);
+            o[i] = make_uint2(p, q);
+            p += c ? 1u : 0u;
+            q += c;
+            if (live && (g & COUNT_LIVE))
+                live[l++] = t0 + i;
+        }
+        if (s.y) {  // some of the four draw
+            uint4 *to = reinterpret_cast<uint4 *>(ex + t0);
+            to[0] = make_uint4(o[0].x, o[0].y, o[1].x, o[1].y);
+            to[1] = make_uint4(o[2].x, o[2].y, o[3].x, o[3].y);
+        }
+        const uint32_t tx = __builtin_amdgcn_readlane(inc.x, 63);
+        run.x += tx & 0xFFFFu;
+        run.y += __builtin_amdgcn_readlane(inc.y, 63);
+        run.z += tx >> 16;
+    }
+    // the appended ones
+    if (!any)
+        return;
+    uint32_t before = 0;  // fans the batch has appended
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+        const uint32_t t0 = b * (uint32_t)BATCH + r * 256 + 4 * lane;
+        const uint32_t fr = f[r];
+        uint2 x[4], s = make_uint2(0u, 0u);  // {fans | drawn ones << 16, pairs}
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = appended(xq[r], fr, i);
+            s = sadd(s, x[i]);
+        }
+        const uint2 inc = wave_incl(s);
+        uint2 at = ssub(inc, s);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if ((fr >> (8 * i)) & COUNT_APPENDS)
+                app_ex[t0 + i] = make_uint4(run.x + (at.x >> 16), run.y + at.y,
+                                            before + (at.x & 0xFFFFu), 0u);
+            at = sadd(at, x[i]);
+        }
+        const uint32_t tx = __builtin_amdgcn_readlane(inc.x, 63);
+        run.x += tx >> 16;
+        run.y += __builtin_amdgcn_readlane(inc.y, 63);
+        before += tx & 0xFFFFu;
+    }
+}
+
+static uint32_t fan_blocks(uint64_t batches)
+{
+    return (uint32_t)((batches + FAN_BATCHES - 1) / FAN_BATCHES);
+}
+
+size_t fan_scan_bytes(uint64_t batches) { return ((size_t)fan_blocks(batches) + 1) * 16; }
+
+// Draws of up to this many workgroups (16k triangles) take one launch: adding up what lies
+// before costs a workgroup at most 48 KB of reads that hit the L2, a launch some 5 us.
+constexpr uint32_t FAN_ONE_PASS = 4;
+
+hipError_t scan_fans(const uint32_t *cnt, const uint8_t *cflag, const uint2 *app, uint2 *ex,
+                     uint4 *app_ex, uint32_t *live, uint64_t batches, void *tmp,
+                     unsigned long long *status, uint64_t cap_prims, uint64_t cap_pairs,
+                     hipStream_t s)
+{
+    if (!batches)
+        return hipSuccess;
+    uint4 *sums = static_cast<uint4 *>(tmp);
+    const uint32_t nb = fan_blocks(batches), n = (uint32_t)batches;
+    const dim3 g(nb), t(SCAN_THREADS);
+    if (nb <= FAN_ONE_PASS) {
+        hipLaunchKernelGGL(k_fan_down<FAN_COUNTS>, g, t, 0, s, cnt, cflag, app, n, sums, ex,
+                           app_ex, live, status, cap_prims, cap_pairs);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(k_fan_reduce, g, t, 0, s, cnt, cflag, app, n, sums);
+    if (nb <= SCAN_CARRY_BLOCKS) {
+        hipLaunchKernelGGL(k_fan_down<FAN_SUMS>, g, t, 0, s, cnt, cflag, app, n, sums, ex,
+                           app_ex, live, status, cap_prims, cap_pairs);
+    } else {
+        hipLaunchKernelGGL(k_scan_sums<uint4>, dim3(1), t, 0, s, sums, nb);
+        hipLaunchKernelGGL(k_fan_down<FAN_SCANNED>, g, t, 0, s, cnt, cflag, app, n, sums, ex,
+                           app_ex, live, status, cap_prims, cap_pairs);
+    }
     return hipGetLastError();
 }
 
