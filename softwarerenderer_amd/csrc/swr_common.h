@@ -174,20 +174,37 @@ __device__ inline bool block_may_cover(const float *e, int x, int y, int ext = 7
     return true;
 }
 
+// Span: a primitive's two flat parts, in registers for walks over several scanlines.
+struct SpanRec {
+    float ox[2], oy[2], is1[2], is2[2];  // bottom-flat, top-flat
+    int lo[2], hi[2];
+};
+
+__device__ inline SpanRec load_span(const float *rec)
+{
+    SpanRec s;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const float *p = rec + (q == 0 ? REC_BOT : REC_TOP);
+        s.ox[q] = p[0];
+        s.oy[q] = p[1];
+        s.is1[q] = p[2];
+        s.is2[q] = p[3];
+        s.lo[q] = (int)__float_as_uint(p[4]);
+        s.hi[q] = (int)__float_as_uint(p[5]);
+    }
+    return s;
+}
+
 // Span: the flat part owning scanline y and its pixel range [xl, xr)
 // (Rasterizer.h:370-380 bottom-flat, :397-407 top-flat).  Returns false when no part owns y.
-__device__ inline bool span_row_extent(const float *rec, uint32_t flags, int y, int sc_minx,
+__device__ inline bool span_row_extent(const SpanRec &s, uint32_t flags, int y, int sc_minx,
                                        int sc_maxx, int &xl, int &xr)
 {
-    const int blo = (int)__float_as_uint(rec[REC_BOT + 4]);
-    const int bhi = (int)__float_as_uint(rec[REC_BOT + 5]);
-    const int tlo = (int)__float_as_uint(rec[REC_TOP + 4]);
-    const int thi = (int)__float_as_uint(rec[REC_TOP + 5]);
-    const bool inb = (flags & FLAG_BOTTOM) && blo <= y && y < bhi;
-    const bool intop = (flags & FLAG_TOP) && tlo < y && y <= thi;
-    const int base = inb ? REC_BOT : REC_TOP;
-    const float ox = rec[base + 0], oy = rec[base + 1];
-    const float is1 = rec[base + 2], is2 = rec[base + 3];
+    const bool inb = (flags & FLAG_BOTTOM) && s.lo[0] <= y && y < s.hi[0];
+    const bool intop = (flags & FLAG_TOP) && s.lo[1] < y && y <= s.hi[1];
+    const float ox = inb ? s.ox[0] : s.ox[1], oy = inb ? s.oy[0] : s.oy[1];
+    const float is1 = inb ? s.is1[0] : s.is1[1], is2 = inb ? s.is2[0] : s.is2[1];
     const float dy = ((float)y - oy) + 0.5f;
     const float cx1 = ox + is1 * dy + 0.5f;
     const float cx2 = ox + is2 * dy + 0.5f;
@@ -196,17 +213,23 @@ __device__ inline bool span_row_extent(const float *rec, uint32_t flags, int y, 
     return inb || intop;
 }
 
-// Span: true when some scanline of the 8x8 block at (bx, by) has pixels of the primitive
-// inside the block's columns (the ranges the rasterizer computes, Rasterizer.h:370-380,
-// 397-407).
-__device__ inline bool span_block_any(const float *rec, uint32_t flags, int bx, int by,
-                                      int sc_minx, int sc_maxx)
+__device__ inline bool span_row_extent(const float *rec, uint32_t flags, int y, int sc_minx,
+                                       int sc_maxx, int &xl, int &xr)
+{
+    return span_row_extent(load_span(rec), flags, y, sc_minx, sc_maxx, xl, xr);
+}
+
+// Span: true when some scanline of the square block of `size` pixels at (bx, by) has pixels of
+// the primitive inside the block's columns (the ranges the rasterizer computes,
+// Rasterizer.h:370-380, 397-407).
+__device__ inline bool span_block_any(const SpanRec &s, uint32_t flags, int bx, int by,
+                                      int sc_minx, int sc_maxx, int size = TILE)
 {
     bool any = false;
-    for (int r = 0; r < TILE && !any; ++r) {
+    for (int r = 0; r < size && !any; ++r) {
         int xl, xr;
-        const bool rowv = span_row_extent(rec, flags, by + r, sc_minx, sc_maxx, xl, xr);
-        any = rowv && imax(xl, bx) < imin(xr, bx + TILE);
+        const bool rowv = span_row_extent(s, flags, by + r, sc_minx, sc_maxx, xl, xr);
+        any = rowv && imax(xl, bx) < imin(xr, bx + size);
     }
     return any;
 }

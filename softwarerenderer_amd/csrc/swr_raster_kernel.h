@@ -378,7 +378,8 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
                                 keep = cls != 0;
                                 pv |= (uint32_t)cls << 30;
                             } else {
-                                keep = span_block_any(rec, flags, bx, by, a.sc_minx, a.sc_maxx);
+                                keep = span_block_any(load_span(rec), flags, bx, by, a.sc_minx,
+                                                      a.sc_maxx);
                             }
                         }
                         // Past a list's first 64 entries, programs that only test z drop what
