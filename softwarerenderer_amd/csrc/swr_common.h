@@ -174,6 +174,65 @@ __device__ inline bool block_may_cover(const float *e, int x, int y, int ext = 7
     return true;
 }
 
+// classify_block's class from which corners pass which edges, in lane masks alone.
+__device__ inline int corners_class(const bool (&p)[4][3])
+{
+    bool any = false, all = true, same = true;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool in = p[q][0] & p[q][1] & p[q][2];
+        any = any | in;
+        all = all & in;
+        same = same & ((p[q][0] == p[q][1]) == p[q][2]);
+    }
+    return any ? (all ? 2 : 1) : (same ? 0 : 1);
+}
+
+// The classes of the 2x2 blocks of the 16-pixel bin at (bx, by), two bits each in row-major
+// order: classify_block of each block of the primitive's block grid, 0 where block_may_cover
+// drops it.  The same operations on the same values, all four blocks and edges without branches,
+// so that the products of a column or row of blocks are taken once and the corners' tests
+// combine in scalar registers (expansion of 1M triangles: 45 -> 29 us; one block at a time is
+// faster the branching way: 244 us against 282 on 12.7M pairs of 8-pixel bins).
+__device__ inline uint32_t classify_blocks4(const float *rec, uint32_t flags, int bx, int by)
+{
+    const uint32_t *ru = reinterpret_cast<const uint32_t *>(rec);
+    const float xf[2] = {(float)bx + 0.5f, (float)(bx + TILE) + 0.5f};
+    const float yf[2] = {(float)by + 0.5f, (float)(by + TILE) + 0.5f}, s = 7.0f;
+    bool p[4][4][3], may[4] = {true, true, true, true};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float a = rec[REC_EDGE + 3 * k], b = rec[REC_EDGE + 3 * k + 1],
+                    c = rec[REC_EDGE + 3 * k + 2];
+        const float ax[2] = {a * xf[0], a * xf[1]}, by2[2] = {b * yf[0], b * yf[1]};
+        const float as = a * s, bs = b * s, span = s * (fabsf(a) + fabsf(b));
+        const float up = fmaxf(0.0f, s * a), vp = fmaxf(0.0f, s * b);
+        const bool tie = (flags >> (1 + k)) & 1u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float x = ax[q & 1], y = by2[q >> 1];
+            const float v00 = x + y + c, v01 = v00 + bs;
+            p[q][0][k] = edge_pass(v00, tie);
+            p[q][1][k] = edge_pass(v01, tie);
+            p[q][2][k] = edge_pass(v00 + as, tie);
+            p[q][3][k] = edge_pass(v01 + as, tie);
+            const float m = fabsf(x) + fabsf(y) + fabsf(c) + span;
+            may[q] = may[q] & !(v00 + up + vp < -m * 3.814697265625e-06f);
+        }
+    }
+    const int kx = bx >> 3, ky = by >> 3;
+    uint32_t packed = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int x = kx + (q & 1), y = ky + (q >> 1);
+        const bool in = (x >= (int)ru[REC_BLOCKS]) & (x <= (int)ru[REC_BLOCKS + 2]) &
+                        (y >= (int)ru[REC_BLOCKS + 1]) & (y <= (int)ru[REC_BLOCKS + 3]);
+        const int cls = corners_class(p[q]);
+        packed |= in & ((cls == 2) | may[q]) ? (uint32_t)cls << (2 * q) : 0u;
+    }
+    return packed;
+}
+
 // Span: a primitive's two flat parts, in registers for walks over several scanlines.
 struct SpanRec {
     float ox[2], oy[2], is1[2], is2[2];  // bottom-flat, top-flat

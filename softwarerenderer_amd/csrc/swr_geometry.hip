@@ -249,6 +249,7 @@ __device__ inline bool prim_geometry(const GeomArgs &a, const WinV &v0, const Wi
 //   Block, other larger bins: dropped when no pixel of the bin can pass all three edge
 //     tests (block_may_cover over the bin); the raster kernel classifies each 8x8 block;
 //   Span: exact, the bin's scanline ranges are those the rasterizer computes.
+template <bool CLS4>
 __device__ inline void pair_for_tile(const GeomArgs &a, const float *rec, uint32_t flags,
                                      uint32_t pos, int tx, int ty, uint32_t &key, uint32_t &val)
 {
@@ -266,33 +267,20 @@ __device__ inline void pair_for_tile(const GeomArgs &a, const float *rec, uint32
     const int size = 1 << a.bin_shift;
     const int bx = tx << a.bin_shift, by = ty << a.bin_shift;
     if (flags & FLAG_BLOCK) {
-        if (size == TILE) {
+        if (!CLS4 && size == TILE) {
             int cls = classify_block(rec + REC_EDGE, flags, bx, by);
             if (cls == 1 && !block_may_cover(rec + REC_EDGE, bx, by))
                 cls = 0;
             key = cls ? key : a.sentinel;
             val |= (uint32_t)cls << 30;
-        } else if (a.cls4) {
-            const uint32_t *ru = reinterpret_cast<const uint32_t *>(rec);
-            uint32_t packed = 0;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int kx = (bx >> 3) + (b & 1), ky = (by >> 3) + (b >> 1);
-                int cls = 0;
-                if (kx >= (int)ru[REC_BLOCKS] && kx <= (int)ru[REC_BLOCKS + 2] &&
-                    ky >= (int)ru[REC_BLOCKS + 1] && ky <= (int)ru[REC_BLOCKS + 3]) {
-                    cls = classify_block(rec + REC_EDGE, flags, kx << 3, ky << 3);
-                    if (cls == 1 && !block_may_cover(rec + REC_EDGE, kx << 3, ky << 3))
-                        cls = 0;
-                }
-                packed |= (uint32_t)cls << (2 * b);
-            }
+        } else if (CLS4) {
+            const uint32_t packed = classify_blocks4(rec, flags, bx, by);
             key = packed ? key : a.sentinel;
             val |= packed << PAIR_CLS4_SHIFT;
         } else {
             key = block_may_cover(rec + REC_EDGE, bx, by, size - 1) ? key : a.sentinel;
         }
-    } else if (a.cls4) {
+    } else if (CLS4) {
         const SpanRec sp = load_span(rec);
         uint32_t packed = 0;
 #pragma unroll
@@ -390,19 +378,32 @@ __device__ __forceinline__ void write_prim(const GeomArgs &a, uint64_t pos, uint
     a.prim_pb[pos] = (uint32_t)pair_base;  // the expansion kernel searches these
 }
 
+// wave-wide inclusive prefix sum
+__device__ inline uint32_t wave_incl_sum(uint32_t x, uint32_t lane)
+{
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1) {
+        const uint32_t o = __shfl_up(x, sh, 64);
+        x += lane >= (uint32_t)sh ? o : 0u;
+    }
+    return x;
+}
+
 // (tile, primitive) pairs, load-balanced: each workgroup owns EXPAND_CHUNK consecutive pair
 // slots (256 to 4096; tunable).  Pair bases are increasing in draw order, so the primitives
 // owning a chunk are a contiguous run found by one binary search; a bit per slot marks where
 // one of them starts, so each thread counts its slot's primitive instead of searching the run,
 // and classifies the slot's tile (row-major rect order).  A Span primitive's parts stay in
-// registers for the tile's scanlines.  Bound by VALU issue (Block: four blocks classified per
-// 16-pixel bin).  64 views of 82k Span triangles: 102 us with a search in LDS and the parts read
-// again for every scanline, 64 us; 150k triangles, Adaptive: 27 -> 24 us; 1M, Block, 16-pixel
-// bins: 45 us both ways.  The tiles the primitive cannot shade are dropped here: the kept pairs are
-// written in slot order to the start of the chunk and their count to chunk_kept[chunk], so
-// the sort reads only kept pairs (without chunk_kept the chunk is written whole, rejected
-// pairs keyed with the sentinel).
-template <int EXPAND_CHUNK>
+// registers for the tile's scanlines.  The tiles the primitive cannot shade are dropped here:
+// the kept pairs are written in slot order to the start of the chunk and their count to
+// chunk_kept[chunk], so the sort reads only kept pairs (without chunk_kept the chunk is written
+// whole, rejected pairs keyed with the sentinel).
+//
+// Bound by VALU issue (the classification).  64 views of 82k Span triangles: 102 us with a
+// search in LDS and the parts read again for every scanline, 65 us now; 150k triangles,
+// Adaptive: 27 -> 23 us; 1M, Block, 16-pixel bins: 45 -> 27 us (classify_blocks4); large Block
+// triangles, whose chunks hold few primitives: 244 us both ways.
+template <int EXPAND_CHUNK, bool CLS4>
 __global__ void __launch_bounds__(256) k_expand(GeomArgs a)
 {
     __shared__ uint32_t s_pb[EXPAND_CHUNK];
@@ -454,25 +455,26 @@ __global__ void __launch_bounds__(256) k_expand(GeomArgs a)
         }
     }
     __syncthreads();
-    const unsigned long long *first = reinterpret_cast<const unsigned long long *>(s_first);
-    uint32_t before = 0;  // first pairs in the earlier rounds' slots (uniform)
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    // lane k: the bits of slots 64 k .. 64 k + 63 and the bits before them
+    static_assert(EXPAND_CHUNK <= 64 * 64, "64 slots per lane");
+    unsigned long long bits = 0;
+    if (lane < EXPAND_CHUNK / 64)
+        bits = reinterpret_cast<const unsigned long long *>(s_first)[lane];
+    const uint32_t bits_n = (uint32_t)__popcll(bits);
+    const uint32_t bits_before = wave_incl_sum(bits_n, lane) - bits_n;
     uint32_t kept = 0;  // pairs kept by the earlier rounds (uniform)
     for (uint64_t r0 = c0; r0 < c1; r0 += 256) {  // blockDim.x == 256
         const uint64_t q = r0 + threadIdx.x;
         uint32_t key = a.sentinel, val = 0;
-        // the slot's primitive: as many after the first as first pairs up to the slot
-        uint32_t lo = before;
-        {
-            const uint32_t wd = (uint32_t)(r0 - c0) / 64;
-            const unsigned long long upto = ~0ull >> (63u - lane);
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                const unsigned long long m = first[wd + k];
-                lo += k < w ? (uint32_t)__popcll(m) : (k == w ? (uint32_t)__popcll(m & upto) : 0u);
-                before += (uint32_t)__popcll(m);
-            }
-        }
+        // the slot's primitive: as many after the first as there are bits up to the slot (the
+        // wave's 64 slots are one lane's bits)
+        const int wd = (int)((uint32_t)(r0 - c0) / 64 + w);
+        const uint32_t b0 = __builtin_amdgcn_readlane((uint32_t)bits, wd),
+                       b1 = __builtin_amdgcn_readlane((uint32_t)(bits >> 32), wd);
+        const uint32_t lo =
+            __builtin_amdgcn_readlane(bits_before, wd) + (b0 & 1u) +
+            __builtin_amdgcn_mbcnt_hi(b1 >> 1, __builtin_amdgcn_mbcnt_lo(b0 >> 1 | b1 << 31, 0u));
         if (q < c1) {
             const uint32_t pos = p0 + lo;
             const uint32_t local = (uint32_t)q - s_pb[lo];
@@ -481,7 +483,7 @@ __global__ void __launch_bounds__(256) k_expand(GeomArgs a)
             const int tx0 = (int)ru[REC_TILES + 0], ty0 = (int)ru[REC_TILES + 1];
             const uint32_t w0 = ru[REC_TILES + 2] - ru[REC_TILES + 0] + 1u;
             const int tx = tx0 + (int)(local % w0), ty = ty0 + (int)(local / w0);
-            pair_for_tile(a, rec, ru[REC_FLAGS], pos, tx, ty, key, val);
+            pair_for_tile<CLS4>(a, rec, ru[REC_FLAGS], pos, tx, ty, key, val);
         }
         if (!a.chunk_kept) {
             if (q < c1) {
@@ -1076,17 +1078,6 @@ struct ClipStage {
     float v[MAX_CLIP][NV];
 };
 
-// wave-wide inclusive prefix sum
-__device__ inline uint32_t wave_incl_sum(uint32_t x, uint32_t lane)
-{
-#pragma unroll
-    for (int sh = 1; sh < 64; sh <<= 1) {
-        const uint32_t o = __shfl_up(x, sh, 64);
-        x += lane >= (uint32_t)sh ? o : 0u;
-    }
-    return x;
-}
-
 __device__ inline WinV shfl_win(const WinV &w, int src)
 {
     WinV r;
@@ -1365,7 +1356,11 @@ static hipError_t launch_expand_ch(const GeomArgs &a, hipStream_t s)
     uint64_t blocks = (a.pair_cap + CH - 1) / CH;
     if (blocks < 1)
         blocks = 1;
-    hipLaunchKernelGGL(k_expand<CH>, dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    // (CLS4 apart: the four blocks' classification holds twice the registers)
+    if (a.cls4)
+        hipLaunchKernelGGL((k_expand<CH, true>), dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_expand<CH, false>), dim3((uint32_t)blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
