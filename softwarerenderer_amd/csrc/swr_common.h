@@ -420,7 +420,7 @@ struct RasterArgs {
     uint32_t nscenes;
     int xcd;                    // 1: tile blocks grouped per XCD
     const TexDev *tex;          // SWR_PS_TEXTURE
-    int fold;                   // 1: an asynchronous draw; its failures go to ST_STICKY
+    int fold;                   // 0 (modules built earlier read it; the sort folds failures)
     const void *user;           // SWR_PS_MODULE: the program's uniforms (device memory)
     int spans;                  // 0: every primitive is a Block primitive (raster mode Block)
     uint32_t *queue;            // persistent raster: RASTER_QUEUES bin-queue heads, zeroed by the

@@ -34,7 +34,7 @@
 // dL/dimage) and k_diff_bwd_edges (the active pairs: what the antialiasing adds),
 // both reading the stored decisions; gradients reach the vertex attributes through b_i,
 // the clip coordinates through D_i (barycentrics) and through t (the silhouette crossing),
-// accumulated per tile in LDS and flushed with float atomics.  A backward whose buffers are
+// gathered in lists in LDS, summed and flushed with float atomics.  A backward whose buffers are
 // not those of the last forward on the context takes decisions again itself
 // (k_diff_backward).  The walk is queued because few pairs need it (about 1% on a
 // 41k-vertex sphere at 512 x 512) and a wave that holds one waits on its chain of dependent
@@ -1411,9 +1411,10 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
 // pixel's half, B is the front pixel and the source the other pixel's colour, else B is the
 // other pixel and the source the silhouette triangle's colour at the crossing.  Either way the
 // source is a triangle's interpolation along a ray, so all lanes run the same code: B's and
-// the source's interpolation, forward and backward, and the crossing's derivatives.  Bound by the latency of that chain
-// (dependent loads, fp64 divisions), so it is kept short and every wave gets 64 pairs: pairs
-// cluster on silhouettes, and a wave per 16 tiles left most waves idle behind a few long ones.
+// the source's interpolation, forward and backward, and the crossing's derivatives.  Bound by the
+// latency of that chain (dependent loads, fp64 divisions), so it is kept short and every wave
+// gets 64 pairs: pairs cluster on silhouettes, and a wave per 16 tiles left most waves idle
+// behind a few long ones.
 // One 256x256 view / 64 views of 512x512 / 16 terrain views of 768x768, beside the interior
 // kernel: 79 / 553 / 1007 us with a lane per pixel and its four pairs in turn, 31 / 67 / 347 us
 // with a lane per pair and a wave per 16 tiles, 20 / 56 / 146 us now.

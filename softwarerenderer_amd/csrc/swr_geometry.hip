@@ -3,8 +3,8 @@
 // One thread per input triangle.  A count pass and an emit pass run the same device code
 // (process_triangle<NV, EMIT>): vertex program, clip masks and Sutherland-Hodgman clipping
 // against the six frustum planes, perspective divide + viewport, facing cull, triangle
-// setup and the tile rectangle each surviving triangle touches.  Between the passes two
-// exclusive scans turn per-triangle counts into draw-order positions, so the emit pass
+// setup and the tile rectangle each surviving triangle touches.  Between the passes a
+// scan turns per-triangle counts into draw-order positions, so the emit pass
 // writes primitive records and (tile, primitive) pairs in the reference's draw order with
 // no sorting and no atomics:
 //   key order = (batch, phase, j, k): per 1024-triangle batch, first triangle j's fan
@@ -14,9 +14,9 @@
 // The vertex cache of the reference (VertexCache.h:29-63, used at VertexProcessor.cpp:86-117)
 // maps an index to an already shaded output vertex within a batch.  Vertex programs are
 // pure, so the results do not depend on which reference to a vertex shades it.  Here the
-// vertex pass (shade_vertex, in the begin kernel) shades every vertex of the attribute buffer once, in index order,
-// into post-transform arrays (window-space position and clip mask), which both geometry
-// passes read by index; the emit pass fetches only the varyings the vertex program copies.
+// vertex pass (shade_vertex, in the begin kernel) shades every vertex of the attribute buffer
+// once, in index order, into post-transform arrays (window-space position and clip mask),
+// which both geometry passes read by index; the emit pass fetches only the varyings the vertex program copies.
 // Triangles with a vertex outside a clip plane (clip mask != 0) re-run the program for the
 // clip-space position the clipper needs.  Without the vertex pass (a batch of scenes, an
 // attribute buffer of unknown size, or the tuning's choice) every corner runs the program.

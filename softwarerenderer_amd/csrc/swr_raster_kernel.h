@@ -240,8 +240,6 @@ __global__ void __launch_bounds__(512) k_raster(RasterArgs a0)
     __shared__ unsigned long long s_cov[NEAREST ? 1 : MAXW][GS];
     __shared__ uint32_t s_ring[RW][RING];
 
-    if (a0.fold && blockIdx.x == 0 && threadIdx.x == 0)
-        fold_status(const_cast<unsigned long long *>(a0.status));
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int wpb = (int)(blockDim.x >> 6);
     // 8x8 blocks per bin side: 1 for 8x8 bins (FILT = false), else 2 or 4
