@@ -107,6 +107,22 @@ __device__ inline void lds_sync()
     __asm__ volatile("" ::: "memory");
 }
 
+// Wave-wide inclusive scan of 64 lanes: DPP steps inside the rows of 16 lanes, then the rows'
+// totals handed on (a shuffle per step waits for the LDS six times over).  Every lane calls it.
+__device__ inline uint32_t wave_incl(uint32_t v)
+{
+#define SWR_SCAN_STEP(CTRL, ROWS) \
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false)
+    SWR_SCAN_STEP(0x111, 0xF);  // row_shr 1, 2, 4, 8
+    SWR_SCAN_STEP(0x112, 0xF);
+    SWR_SCAN_STEP(0x114, 0xF);
+    SWR_SCAN_STEP(0x118, 0xF);
+    SWR_SCAN_STEP(0x142, 0xA);  // row_bcast 15, 31
+    SWR_SCAN_STEP(0x143, 0xC);
+#undef SWR_SCAN_STEP
+    return v;
+}
+
 // EdgeEquation::test (EdgeEquation.h:53-61): v > 0 || (v == 0 && tie), as one compare:
 // v >= 0 with the tie, v >= the smallest denormal without it (the kernels keep fp32
 // denormals, so nothing lies strictly between 0 and it; NaN fails both forms).

@@ -378,17 +378,6 @@ __device__ __forceinline__ void write_prim(const GeomArgs &a, uint64_t pos, uint
     a.prim_pb[pos] = (uint32_t)pair_base;  // the expansion kernel searches these
 }
 
-// wave-wide inclusive prefix sum
-__device__ inline uint32_t wave_incl_sum(uint32_t x, uint32_t lane)
-{
-#pragma unroll
-    for (int sh = 1; sh < 64; sh <<= 1) {
-        const uint32_t o = __shfl_up(x, sh, 64);
-        x += lane >= (uint32_t)sh ? o : 0u;
-    }
-    return x;
-}
-
 // (tile, primitive) pairs, load-balanced: each workgroup owns EXPAND_CHUNK consecutive pair
 // slots (256 to 4096; tunable).  Pair bases are increasing in draw order, so the primitives
 // owning a chunk are a contiguous run found by one binary search; a bit per slot marks where
@@ -462,7 +451,7 @@ __global__ void __launch_bounds__(256) k_expand(GeomArgs a)
     if (lane < EXPAND_CHUNK / 64)
         bits = reinterpret_cast<const unsigned long long *>(s_first)[lane];
     const uint32_t bits_n = (uint32_t)__popcll(bits);
-    const uint32_t bits_before = wave_incl_sum(bits_n, lane) - bits_n;
+    const uint32_t bits_before = wave_incl(bits_n) - bits_n;
     uint32_t kept = 0;  // pairs kept by the earlier rounds (uniform)
     for (uint64_t r0 = c0; r0 < c1; r0 += 256) {  // blockDim.x == 256
         const uint64_t q = r0 + threadIdx.x;
@@ -1222,7 +1211,7 @@ __device__ void clip_queued(const GeomArgs &a0, uint32_t t, ClipStage<NV> &st)
     }
     const unsigned long long m_drawn = __ballot(drawn);
     const uint32_t nt1 = lane >= 1 ? nt : 0u;  // pairs of the appended fans
-    const uint32_t incl = wave_incl_sum(nt1, lane);
+    const uint32_t incl = wave_incl(nt1);
     if (!EMIT) {
         const uint32_t tot1 = __shfl(incl, 63);
         if (lane == 0) {
@@ -1259,7 +1248,7 @@ __device__ void run_clip_queue(const GeomArgs &a, uint32_t wid, uint32_t nwaves,
         // the 64 counters load in parallel, one per lane; an inclusive scan across the wave
         const uint32_t lane = threadIdx.x & 63u;
         const uint32_t cnt = a.clipq_cnt[lane * CLIPQ_STRIDE];
-        const uint32_t incl = wave_incl_sum(cnt, lane);
+        const uint32_t incl = wave_incl(cnt);
         s_off[lane] = incl - cnt;
         if (lane == 63)
             s_off[CLIPQ_REGIONS] = incl;

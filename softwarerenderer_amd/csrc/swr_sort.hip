@@ -36,21 +36,6 @@ template <> __device__ inline uint32_t szero<uint32_t>() { return 0u; }
 template <> __device__ inline uint2 szero<uint2>() { return make_uint2(0u, 0u); }
 template <> __device__ inline uint4 szero<uint4>() { return make_uint4(0u, 0u, 0u, 0u); }
 
-// Wave-wide inclusive scan of 64 lanes: DPP steps inside the rows of 16 lanes, then the rows'
-// totals handed on (a shuffle per step waits for the LDS six times over).
-__device__ inline uint32_t wave_incl(uint32_t v)
-{
-#define SWR_SCAN_STEP(CTRL, ROWS) \
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false)
-    SWR_SCAN_STEP(0x111, 0xF);  // row_shr 1, 2, 4, 8
-    SWR_SCAN_STEP(0x112, 0xF);
-    SWR_SCAN_STEP(0x114, 0xF);
-    SWR_SCAN_STEP(0x118, 0xF);
-    SWR_SCAN_STEP(0x142, 0xA);  // row_bcast 15, 31
-    SWR_SCAN_STEP(0x143, 0xC);
-#undef SWR_SCAN_STEP
-    return v;
-}
 __device__ inline uint2 wave_incl(uint2 v) { return make_uint2(wave_incl(v.x), wave_incl(v.y)); }
 __device__ inline uint4 wave_incl(uint4 v)
 {
