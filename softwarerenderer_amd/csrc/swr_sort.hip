@@ -3,9 +3,9 @@
 // Binning needs, per 8x8 tile, the primitives touching it in draw order.  The emit pass
 // writes (tile, primitive) pairs grouped by primitive in draw order; a stable radix sort on
 // the tile id regroups them by tile while keeping draw order inside each tile.  Only each
-// tile's own order matters, not the order of the tiles, so one scatter by the id's low 8 bits
-// makes 256 buckets, and one workgroup per bucket regroups its pairs by the remaining bits
-// and writes its tiles' ranges (k_bucket; up to 2^18 tiles).  More tiles take least
+// tile's own order matters, not the order of the tiles, so one scatter deals the ids to 256
+// buckets (swr_buckets.h), and one workgroup per bucket regroups its pairs by the ids' remaining
+// bits and writes its tiles' ranges (k_bucket; up to 2^18 tiles).  More tiles take least
 // significant digit passes of 8 bits each, then k_ranges.  Ranks inside a block are made
 // stable with wave ballots: the lanes of a wave holding the same digit are found with a
 // ballot per bit, and a lane's rank is the number of such lanes below it.
@@ -16,6 +16,7 @@
 // 8160 bins) and 20 instead of 34 us on a small frame (7.5k pairs in 4800 bins).
 #include <utility>
 
+#include "swr_buckets.h"
 #include "swr_common.h"
 #include "swr_internal.h"
 
@@ -656,8 +657,9 @@ __device__ inline uint64_t chunk_slot(const Chunks &ch, uint64_t g0, uint32_t nk
 
 __global__ void __launch_bounds__(RADIX_THREADS) k_radix_hist(const uint32_t *keys,
                                                             const unsigned long long *status,
-                                                            int word, int shift, uint32_t tiles,
-                                                            uint32_t *hist, Chunks ch, int rows)
+                                                            int word, TileDigit digit,
+                                                            uint32_t tiles, uint32_t *hist,
+                                                            Chunks ch, int rows)
 {
     __shared__ uint32_t h[256];
     __shared__ uint32_t s_off[RADIX_THREADS + 1];
@@ -673,7 +675,7 @@ __global__ void __launch_bounds__(RADIX_THREADS) k_radix_hist(const uint32_t *ke
             for (uint32_t v = threadIdx.x; v < tot; v += RADIX_THREADS) {
                 const uint32_t k = keys[chunk_slot(ch, g0, nk, s_off, v)];
                 if (k < tiles)
-                    atomicAdd(&h[(k >> shift) & 255u], 1u);
+                    atomicAdd(&h[digit.of(k)], 1u);
             }
             __syncthreads();  // s_off is reloaded by the next group
         }
@@ -683,7 +685,7 @@ __global__ void __launch_bounds__(RADIX_THREADS) k_radix_hist(const uint32_t *ke
         for (uint64_t i = beg + threadIdx.x; i < end; i += RADIX_THREADS) {
             uint32_t k = keys[i];
             if (k < tiles)
-                atomicAdd(&h[(k >> shift) & 255u], 1u);
+                atomicAdd(&h[digit.of(k)], 1u);
         }
     }
     __syncthreads();
@@ -726,8 +728,8 @@ constexpr int RADIX_ITEMS = 4;
 // slot slot_of(i); run[] carries each digit's next output position between rounds.
 template <class SlotOf>
 __device__ inline void scatter_round(const uint32_t *keys, const uint32_t *vals, uint32_t *okeys,
-                                     uint32_t *ovals, int shift, uint32_t tiles, uint64_t cap,
-                                     uint64_t base, uint64_t end, SlotOf slot_of, uint32_t *run,
+                                     uint32_t *ovals, TileDigit digit, uint32_t tiles,
+                                     uint64_t cap, uint64_t base, uint64_t end, SlotOf slot_of, uint32_t *run,
                                      uint32_t (*wcnt)[RADIX_THREADS / 64][256],
                                      uint32_t (*off)[RADIX_THREADS / 64][256])
 {
@@ -744,7 +746,7 @@ __device__ inline void scatter_round(const uint32_t *keys, const uint32_t *vals,
             k[j] = i < end ? keys[slot] : 0u;
             valid[j] = i < end && k[j] < tiles;
             v[j] = valid[j] ? vals[slot] : 0u;
-            d[j] = (k[j] >> shift) & 255u;
+            d[j] = digit.of(k[j]);
         }
 #pragma unroll
         for (int j = 0; j < RADIX_ITEMS; ++j) {
@@ -787,7 +789,7 @@ __device__ inline void scatter_round(const uint32_t *keys, const uint32_t *vals,
 
 __global__ void __launch_bounds__(RADIX_THREADS) k_radix_scatter(
     const uint32_t *keys, const uint32_t *vals, uint32_t *okeys, uint32_t *ovals,
-    unsigned long long *status, int word, int shift, uint32_t tiles, const uint32_t *hist,
+    unsigned long long *status, int word, TileDigit digit, uint32_t tiles, const uint32_t *hist,
     uint32_t *tot, Chunks ch, int rows)
 {
     constexpr int NW = RADIX_THREADS / 64;
@@ -838,7 +840,7 @@ __global__ void __launch_bounds__(RADIX_THREADS) k_radix_scatter(
             const uint32_t nk = load_chunk_group(ch, g0, k1, s_off);
             const uint32_t tot = s_off[RADIX_THREADS];
             for (uint64_t base = 0; base < tot; base += (uint64_t)RADIX_THREADS * RADIX_ITEMS)
-                scatter_round(keys, vals, okeys, ovals, shift, tiles, cap, base, tot,
+                scatter_round(keys, vals, okeys, ovals, digit, tiles, cap, base, tot,
                               [&](uint64_t i) { return chunk_slot(ch, g0, nk, s_off, (uint32_t)i); },
                               run, wcnt, off);
             __syncthreads();  // s_off is reloaded by the next group
@@ -847,18 +849,18 @@ __global__ void __launch_bounds__(RADIX_THREADS) k_radix_scatter(
         uint64_t beg, end;
         chunk_of(status, word, G, b, beg, end);
         for (uint64_t base = beg; base < end; base += (uint64_t)RADIX_THREADS * RADIX_ITEMS)
-            scatter_round(keys, vals, okeys, ovals, shift, tiles, cap, base, end,
+            scatter_round(keys, vals, okeys, ovals, digit, tiles, cap, base, end,
                           [](uint64_t i) { return i; }, run, wcnt, off);
     }
 }
 
-// One bucket: the pairs whose tile id has low byte blockIdx.x, a run of the scatter's output
-// (tot: the buckets' lengths).  Each wave owns a contiguous piece of the run: it counts its
-// pairs per tile (the id's bits above the low 8: `bits` of them), the counts of all waves
-// scanned tile by tile give every (wave, tile) its first position, and the wave walks its
+// One bucket: the pairs of the tiles that swr_buckets.h deals to bucket blockIdx.x, a run of the
+// scatter's output (tot: the buckets' lengths).  Each wave owns a contiguous piece of the run: it
+// counts its pairs per tile (the id's bits above the low 8: `bits` of them), the counts of all
+// waves scanned tile by tile give every (wave, tile) its first position, and the wave walks its
 // piece again, placing its pairs in order.  The tiles' ranges are written whether they hold
-// pairs or not.  Runs differ in length with the picture, neighbouring tiles lie in different
-// buckets.
+// pairs or not.  A bucket's time grows with its run, so the runs must not differ much: tiles
+// that lie together on the screen lie in different buckets.
 __global__ void __launch_bounds__(1024) k_bucket(const uint32_t *keys, const uint32_t *vals,
                                                  uint32_t *ovals, unsigned long long *status,
                                                  const uint32_t *tot, int bits, uint32_t tiles,
@@ -919,7 +921,7 @@ __global__ void __launch_bounds__(1024) k_bucket(const uint32_t *keys, const uin
                 sum += s_cnt[(q << bits) + v];
         uint32_t at = base + block_excl(sum, &all);
         if (v < nv) {
-            const uint32_t tile = (v << 8) | bucket;
+            const uint32_t tile = bucket_tile(bucket, v);
             if (tile < tiles) {
                 ranges[2 * (size_t)tile] = at;
                 ranges[2 * (size_t)tile + 1] = at + sum;
@@ -1010,17 +1012,17 @@ hipError_t sort_pairs(SortBuffers &sb, unsigned long long *status, uint32_t tile
     uint32_t *ka = sb.keys_a, *va = sb.vals_a, *kb = sb.keys_b, *vb = sb.vals_b;
     const int rows = sb.blocks <= SCAN_ROWS ? 1 : 0;
     for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
+        const TileDigit digit = {8 * p, bucket};
         const int word = p == 0 ? ST_PAIRS : ST_KEPT;
         // pass 0 reads the expansion's chunks (when it compacted them), later passes one run
         Chunks ch{p == 0 ? sb.chunk_kept : nullptr, sb.chunk};
         hipLaunchKernelGGL(k_radix_hist, dim3(sb.blocks), dim3(RADIX_THREADS), 0, s, ka, status,
-                           word, shift, tiles, sb.hist, ch, rows);
+                           word, digit, tiles, sb.hist, ch, rows);
         if (!rows)
             hipLaunchKernelGGL(k_radix_scan, dim3(256), dim3(RADIX_THREADS), 0, s, sb.hist,
                                sb.blocks, sb.tot);
         hipLaunchKernelGGL(k_radix_scatter, dim3(sb.blocks), dim3(RADIX_THREADS), 0, s, ka, va, kb,
-                           vb, status, word, shift, tiles, sb.hist, sb.tot, ch, rows);
+                           vb, status, word, digit, tiles, sb.hist, sb.tot, ch, rows);
         std::swap(ka, kb);
         std::swap(va, vb);
     }
