@@ -10,7 +10,7 @@
 // times by the low bits; constant steps from run to run meet widths and slopes at which it holds
 // 16 to 255 times its share.  300,000 triangles in a column of 8 pixels of a 2048x2048 target:
 // 805 us a draw by the low bits, 588 us with digit passes instead of buckets, 438 us so; in 64
-// columns 252, 248 and 199 us; draws spread over the screen take the same either way.
+// columns of pixels 252, 248 and 199 us; draws spread over the screen take the same either way.
 #pragma once
 
 #include <stdint.h>

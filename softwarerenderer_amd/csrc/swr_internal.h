@@ -38,6 +38,7 @@ struct LineArgs {
     float *frags;           // fragment records (emit pass)
     int fstride;            // words per fragment record
     uint32_t *keys, *vals;  // (tile, fragment) pairs in fragment order
+    uint32_t group0;        // the first workgroup of a later launch (set by the launchers)
 };
 int fragment_stride(const ParamLayout &L);
 uint32_t lines_groups(uint64_t prims);

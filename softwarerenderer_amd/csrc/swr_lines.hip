@@ -215,15 +215,16 @@ __device__ inline void write_fragment(const LineArgs &A, uint64_t f, uint64_t i,
 // two words, now 6 us.
 constexpr uint32_t LINE_PIECE = 32, LINES = 16;
 
-template <int NV, bool EMIT>
+// FAR: a launch of later workgroups, from A.group0 on (launch_walk).
+template <int NV, bool EMIT, bool FAR>
 __global__ void __launch_bounds__(64) k_lines_walk(LineArgs A)
 {
     constexpr int W = 4 + NV, ST = 2 * W + 1;  // start and step; odd: lines spread over banks
     __shared__ float s_line[LINES * ST];
     __shared__ uint32_t s_steps[LINES], s_first[LINES], s_done[LINES];
     const GeomArgs &a = A.g;
-    const uint32_t lane = threadIdx.x;
-    const uint64_t base = (uint64_t)blockIdx.x * LINES, i = base + lane;
+    const uint32_t lane = threadIdx.x, group = (FAR ? A.group0 : 0u) + blockIdx.x;
+    const uint64_t base = (uint64_t)group * LINES, i = base + lane;
     LVert<NV> V[2];
     const bool mine = lane < LINES && i < A.prims;
     bool live = mine && (!EMIT || A.count[i].y != 0u) && prepare_primitive<NV>(A, i, V);
@@ -370,7 +371,7 @@ __global__ void __launch_bounds__(64) k_lines_walk(LineArgs A)
         // fit 32 bits, all of them need not)
         const unsigned long long frags = wave_sum(n);
         if (lane == 0)
-            A.parts[blockIdx.x] = frags;
+            A.parts[group] = frags;
     }
 }
 
@@ -386,28 +387,37 @@ __global__ void __launch_bounds__(256) k_lines_begin(LineArgs A)
 // ---- launchers ------------------------------------------------------------------------------
 uint32_t lines_groups(uint64_t prims) { return (uint32_t)((prims + LINES - 1) / LINES); }
 
+// A launch holds fewer than 2^32 threads, which 2^30 primitives, the most a draw takes, reach
+// with 4 threads each: a second launch takes the workgroups from 2^25 on (an offset in every
+// launch costs long lines 2%).
+template <int NV, bool EMIT>
+static void launch_walk(LineArgs A, hipStream_t s)
+{
+    const uint32_t n = lines_groups(A.prims), most = 1u << 25, first = n < most ? n : most;
+    if (first)
+        hipLaunchKernelGGL((k_lines_walk<NV, EMIT, false>), dim3(first), dim3(64), 0, s, A);
+    A.group0 = first;
+    if (n > first)
+        hipLaunchKernelGGL((k_lines_walk<NV, EMIT, true>), dim3(n - first), dim3(64), 0, s, A);
+}
+
 hipError_t launch_lines_count(const LineArgs &A, hipStream_t s)
 {
     const uint64_t clear = A.g.tiles * 2ull > ST_WORDS ? A.g.tiles * 2ull : ST_WORDS;
     const uint64_t cb = (clear + 255) / 256 < 4096 ? (clear + 255) / 256 : 4096;
     hipLaunchKernelGGL(k_lines_begin, dim3((uint32_t)cb), dim3(256), 0, s, A);
-    if (A.prims)
-        hipLaunchKernelGGL((k_lines_walk<0, false>), dim3(lines_groups(A.prims)), dim3(64), 0, s,
-                           A);
+    launch_walk<0, false>(A, s);
     return hipGetLastError();
 }
 
 hipError_t launch_lines_emit(const LineArgs &A, hipStream_t s)
 {
-    if (!A.prims)
-        return hipSuccess;
-    const dim3 g(lines_groups(A.prims)), b(64);
     switch (emit_class(A.g.lay.na + A.g.lay.np)) {
-    case 0: hipLaunchKernelGGL((k_lines_walk<0, true>), g, b, 0, s, A); break;
-    case 3: hipLaunchKernelGGL((k_lines_walk<3, true>), g, b, 0, s, A); break;
-    case 5: hipLaunchKernelGGL((k_lines_walk<5, true>), g, b, 0, s, A); break;
-    case 8: hipLaunchKernelGGL((k_lines_walk<8, true>), g, b, 0, s, A); break;
-    default: hipLaunchKernelGGL((k_lines_walk<32, true>), g, b, 0, s, A); break;
+    case 0: launch_walk<0, true>(A, s); break;
+    case 3: launch_walk<3, true>(A, s); break;
+    case 5: launch_walk<5, true>(A, s); break;
+    case 8: launch_walk<8, true>(A, s); break;
+    default: launch_walk<32, true>(A, s); break;
     }
     return hipGetLastError();
 }
