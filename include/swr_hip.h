@@ -402,7 +402,8 @@ typedef struct swr_tuning {
     int32_t raster_group;    /* primitives per row-walk group in the raster kernel of the
                                 depth-checker and visibility programs: 1, 2, 4, 8 (program's) */
     int32_t xcd_order;       /* 1: raster tile blocks grouped per XCD (default), -1: linear */
-    int32_t expand_chunk;    /* tile pairs per expansion workgroup: 256 .. 4096 (1024) */
+    int32_t expand_chunk;    /* tile pairs per expansion workgroup: 256 .. 4096 (256 while the
+                                context's pair arena holds up to 2^20 pairs, else 1024) */
     int32_t vertex_pass;     /* 1: shade every vertex of attribute 0 once into post-transform
                                 vertices, -1: shade each triangle corner where it is used,
                                 0: automatic (the pass when the buffer's vertex count is known

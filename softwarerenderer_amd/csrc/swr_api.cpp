@@ -457,14 +457,18 @@ uint32_t sort_blocks(uint64_t pair_cap)
 size_t hist_bytes(uint32_t G) { return (size_t)256 * (G + 1) * 4; }
 // kept-pair counts of the expansion chunks (256 slots at the least)
 size_t chunk_kept_bytes(uint64_t pair_cap) { return (pair_cap / 256 + 1) * 4; }
-// The expansion chunk of a draw: the tuned one, else 1024, or 256 where the pair arena is small:
-// up to 2^17 pairs make at most 128 workgroups of 1024, each a chain of four rounds of dependent
-// loads, while 512 of one round still fit the GPU at once: the VGA sphere, 9,262 pairs: 16 -> 6 us.
+// The expansion chunk of a draw: the tuned one, else 256 where the pair arena holds up to 2^20
+// pairs and 1024 where it holds more.  A workgroup of 1024 is a chain of four rounds of dependent
+// loads, so small draws want many of one round; but the launch covers the arena, whatever part of
+// it the draw fills (the host does not know its pairs), and the sort reads a count per chunk.  Per
+// draw, chunks of 256 against 1024: a VGA sphere, 11k pairs, 53 and 60 us in an arena of 2^17, 55
+// and 62 of 2^20, 69 and 65 of 2^24; 0.7M pairs 135 and 139 us, 1.1M 169 and 168 us, 5.1M 280 and
+// 264 us.
 int expand_chunk_of(int tuned, uint64_t pair_cap)
 {
     if (tuned == 256 || tuned == 512 || tuned == 2048 || tuned == 4096)
         return tuned;
-    return tuned == 0 && pair_cap <= (1u << 17) ? 256 : 1024;
+    return tuned == 0 && pair_cap <= (1u << 20) ? 256 : 1024;
 }
 
 // ---- the no-allocation draw's scratch ------------------------------------------------------
