@@ -31,12 +31,13 @@ SHAPES = ([dict(bin_size=8, raster_waves=w) for w in (1, 2, 4, 8)] +
           [dict(bin_size=b, waves_per_bin=w) for b in (16, 32) for w in (1, 2, 4)])
 VERTEX_PASS = (1, -1)
 # stage 2, for the fastest shape: primitives per raster row-walk group (0: the pixel
-# program's default), XCD-grouped bin order on/off, tile pairs per expansion workgroup,
-# persistent raster workgroups fed by per-XCD bin queues on/off
+# program's default), XCD-grouped bin order on/off, tile pairs per expansion workgroup (0: the
+# built-in rule, 256 for small pair arenas, else 1024), persistent raster workgroups fed by
+# per-XCD bin queues on/off
 REFINE = {
     "raster_group": (0, 1, 2, 4),
     "xcd_order": (1, -1),
-    "expand_chunk": (512, 1024, 2048),
+    "expand_chunk": (0, 512, 2048),
     "raster_queue": (-1, 1),
 }
 
