@@ -1683,20 +1683,10 @@ __global__ void __launch_bounds__(256) k_diff_reduce_attr(DiffArgs d, int C)
     }
 }
 
-// The backward's interior and antialiasing kernels add into the same gradients (commutative
-// atomics) and read nothing the other writes, so with a second stream they run side by side:
-// the interior kernel is bound by LDS atomics, the edge kernel by its arithmetic.  Below
-// SIDE_MIN_TILES tiles (a few 512x512 views) the fork and join cost more than the overlap.
-constexpr uint32_t SIDE_MIN_TILES = 8192;
-struct SideStream {
-    hipStream_t s = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
-};
-
 constexpr uint32_t EDGE_WAVES = 2048;
 
 template <int C>
-static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const SideStream &side)
+static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s)
 {
     const uint32_t blocks = (uint32_t)((size_t)d.tiles_per_view * d.V);
     if (!blocks)
@@ -1708,28 +1698,14 @@ static hipError_t launch_diff(const DiffArgs &d, int which, hipStream_t s, const
         hipLaunchKernelGGL(k_diff_blend<C>, dim3(blocks), dim3(256), 0, s, d);
     } else {
         if (d.pairs == 2) {
-            hipStream_t se = s;
-            const bool fork = side.s && blocks >= SIDE_MIN_TILES;
-            if (fork) {
-                hipError_t e = hipEventRecord(side.fork, s);
-                if (e == hipSuccess)
-                    e = hipStreamWaitEvent(side.s, side.fork, 0);
-                if (e != hipSuccess)
-                    return e;
-                se = side.s;
-            }
+            // Both kernels add into the same gradients and neither reads what the other writes,
+            // but side by side on two streams they are no faster: each fills the GPU, so 64 views
+            // of 512x512 take 1178 us forked and 1173 in turn, 8 views 280 and 266 us.
             // as many waves as the GPU holds (two per SIMD), or a wave per 64 possible pairs
             const uint32_t waves = blocks < EDGE_WAVES / 8 ? blocks * 8 : EDGE_WAVES;
-            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3(waves), dim3(64), 0, se, d,
+            hipLaunchKernelGGL(k_diff_bwd_edges<C>, dim3(waves), dim3(64), 0, s, d,
                                (blocks + d.region_tiles - 1) / d.region_tiles);
             hipLaunchKernelGGL(k_diff_bwd_interior<C>, dim3(blocks), dim3(256), 0, s, d);
-            if (fork) {
-                hipError_t e = hipEventRecord(side.join, side.s);
-                if (e == hipSuccess)
-                    e = hipStreamWaitEvent(s, side.join, 0);
-                if (e != hipSuccess)
-                    return e;
-            }
         } else {
             hipLaunchKernelGGL(k_diff_backward<C>, dim3(blocks), dim3(256), 0, s, d);
         }
@@ -1884,15 +1860,12 @@ static int diff_run(swr_context *c, const swr_diff_desc *dd, const float *gimage
         d.pairs = std::memcmp(held, tag, sizeof tag) == 0 ? 2 : 0;
     }
     hipStream_t s = context_stream(c);
-    SideStream side;
-    if (!context_side(c, &side.s, &side.fork, &side.join))
-        side = SideStream();
     hipError_t e;
     switch (q.channels) {
-    case 1: e = launch_diff<1>(d, which, s, side); break;
-    case 2: e = launch_diff<2>(d, which, s, side); break;
-    case 3: e = launch_diff<3>(d, which, s, side); break;
-    default: e = launch_diff<4>(d, which, s, side); break;
+    case 1: e = launch_diff<1>(d, which, s); break;
+    case 2: e = launch_diff<2>(d, which, s); break;
+    case 3: e = launch_diff<3>(d, which, s); break;
+    default: e = launch_diff<4>(d, which, s); break;
     }
     if (e != hipSuccess)
         return context_fail(c, SWR_ERR_HIP, hipGetErrorString(e));
