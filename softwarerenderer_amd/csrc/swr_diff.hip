@@ -854,13 +854,8 @@ __device__ inline void group_segments(const uint32_t *cnt, uint32_t tiles, uint3
     static_assert(TILES <= 64, "a tile per lane of the first wave");
     if (threadIdx.x < 64) {
         const uint32_t lane = threadIdx.x;
-        uint32_t v = lane < TILES && t0 + lane < tiles ? cnt[t0 + lane] : 0u;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(v, o, 64);
-            if ((int)lane >= o)
-                v += u;
-        }
+        const uint32_t v =
+            wave_incl(lane < TILES && t0 + lane < tiles ? cnt[t0 + lane] : 0u);
         if (lane < TILES)
             s_off[lane + 1] = v;
         if (lane == 0)
@@ -1613,12 +1608,7 @@ __global__ void __launch_bounds__(64) k_diff_bwd_edges(DiffArgs d, uint32_t regi
 #pragma unroll
     for (uint32_t q = 0; q < EDGE_REGIONS / 64; ++q) {
         const uint32_t r = q * 64 + lane;
-        uint32_t c = r < regions ? d.ecnt[r] : 0u, v = c;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(v, o, 64);
-            v += (int)lane >= o ? u : 0u;
-        }
+        const uint32_t c = r < regions ? d.ecnt[r] : 0u, v = wave_incl(c);
         s_off[r] = n + v - c;
         n += __shfl(v, 63, 64);
     }

@@ -266,12 +266,7 @@ __global__ void __launch_bounds__(64) k_lines_walk(LineArgs A)
         }
     }
     const uint32_t pieces = (steps + LINE_PIECE - 1) / LINE_PIECE;
-    uint32_t incl = pieces;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(incl, o, 64);
-        incl += (int)lane >= o ? u : 0u;
-    }
+    const uint32_t incl = wave_incl(pieces);
     if (lane < LINES) {
         s_steps[lane] = steps;
         s_first[lane] = incl - pieces;
@@ -313,12 +308,7 @@ __global__ void __launch_bounds__(64) k_lines_walk(LineArgs A)
         }
         // the piece's first fragment: the line's, plus its earlier pieces' (in this round: the
         // lanes below with the same line)
-        uint32_t ex = cnt;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(ex, o, 64);
-            ex += (int)lane >= o ? u : 0u;
-        }
+        const uint32_t ex = wave_incl(cnt);
         const uint32_t head = s_first[lo] > p0 ? s_first[lo] - p0 : 0u;  // the line's first lane
         const uint32_t before = (uint32_t)__shfl((int)(ex - cnt), (int)head, 64);
         const uint32_t done = s_done[lo];

@@ -618,12 +618,7 @@ __device__ inline uint32_t load_chunk_group(const Chunks &ch, uint64_t g0, uint6
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
     __shared__ uint32_t s_w[RADIX_THREADS / 64];
     const uint32_t c = tid < nk ? ch.kept[g0 + tid] : 0u;
-    uint32_t inc = c;
-#pragma unroll
-    for (int sh = 1; sh < 64; sh <<= 1) {
-        const uint32_t o = __shfl_up(inc, sh, 64);
-        inc += lane >= (uint32_t)sh ? o : 0u;
-    }
+    const uint32_t inc = wave_incl(c);
     if (lane == 63)
         s_w[w] = inc;
     __syncthreads();
