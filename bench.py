@@ -128,7 +128,7 @@ def measured_traffic(workload: str, tuning: dict):
 
 def valu_issue(workload: str, tuning: dict, raster_ms: float):
     """The raster kernel's VALU issue rate: SQ_INSTS_VALU per launch (rocprofv3) over the
-    launch time measured here, against the wave64 fp32 issue peak."""
+    launch time measured here, against the rate of plain fp32 additions recorded with them."""
     t = _counters_for(workload, tuning)
     insts, peak = t.get("valu_insts_per_launch"), t.get("valu_peak_winst_per_s")
     if not insts or not peak or raster_ms <= 0:

@@ -350,7 +350,8 @@ int  swr_batch_destroy(swr_batch *batch);
  *             summed over views to grad_attributes ([vertex_count][channels]).
  * All buffers are device memory; both calls only enqueue kernels on the context stream
  * (they can be captured into a HIP graph).  The backward pass recomputes everything else
- * from ids, depth, bary and color.
+ * from ids, depth, clip and attributes (and color, where the caller keeps one); bary is an
+ * output that nothing here reads again.
  *
  * Several meshes in one call (scenes > 1): scene s owns views scene_views[s] ..
  * scene_views[s+1]-1, vertices scene_vertices[s] .. scene_vertices[s+1]-1 and triangles
@@ -380,7 +381,7 @@ typedef struct swr_diff_desc {
     const float    *attributes;    /* [vertex_count][channels]                             */
     const uint32_t *ids;           /* [views][height][width]: triangle + 1, 0 = background */
     const float    *depth;         /* [views][height][width]                               */
-    float *bary;                   /* [views][height][width][2]: forward out, backward in  */
+    float *bary;                   /* [views][height][width][2]: forward out (required)    */
     float *color;                  /* optional [views][height][width][channels]: forward out,
                                       the colour before antialiasing (NULL: not written; the
                                       kernels recompute the few they need)                 */

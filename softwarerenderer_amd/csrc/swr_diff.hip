@@ -42,9 +42,10 @@
 //
 // Precision.  D_i is a cancellation-prone quantity: for a small or grazing triangle the
 // three clip vectors are nearly parallel, and fp32 loses up to 1e-4 of D.  The values
-// (D, b, t and every derivative) are therefore evaluated in fp64 from the fp32 inputs; the
-// kernels are bound by memory and atomics, not by the fp64 rate.  The discrete choices of
-// the antialiasing pass use fp32, so they are reproducible by a CPU restatement.
+// (D, b, t and every derivative) are therefore evaluated in fp64 from the fp32 inputs.  That
+// arithmetic with its loads is about half of the interior backward (136 of 240 us on 64 views of
+// 512x512) and little of the other kernels, which wait on dependent loads.  The discrete choices
+// of the antialiasing pass use fp32, so they are reproducible by a CPU restatement.
 #include <cstring>
 #include <vector>
 
@@ -1273,8 +1274,8 @@ __device__ inline int row_prev(int v, int edge)
 // that the chains of reads overlap), adds in fp64 and flushes: neighbouring lanes add to
 // neighbouring words of a gradient row, a third of the memory requests of a lane per vertex.
 // Tiles of background alone leave at once.  64 views of 512x512 (41k vertices): 485 us with LDS
-// float atomics and a flush of one lane per vertex, 427 us with lists and that flush, 252 us
-// now (136 us without any accumulation); 16 terrain views of 768x768: 494 -> 346 us.
+// float atomics and a flush of one lane per vertex, 427 us with lists and that flush, 240 us
+// now (136 us without any accumulation); 16 terrain views of 768x768: 189 us.
 constexpr uint32_t LIST_END = 0xFFFFu;
 
 template <int C>
@@ -1410,9 +1411,10 @@ __global__ void __launch_bounds__(256) k_diff_bwd_interior(DiffArgs d)
 // latency of that chain (dependent loads, fp64 divisions), so it is kept short and every wave
 // gets 64 pairs: pairs cluster on silhouettes, and a wave per 16 tiles left most waves idle
 // behind a few long ones.
-// One 256x256 view / 64 views of 512x512 / 16 terrain views of 768x768, beside the interior
-// kernel: 79 / 553 / 1007 us with a lane per pixel and its four pairs in turn, 31 / 67 / 347 us
-// with a lane per pair and a wave per 16 tiles, 20 / 56 / 146 us now.
+// One 256x256 view / 64 views of 512x512 / 16 terrain views of 768x768: 79 / 553 / 1007 us with a
+// lane per pixel and its four pairs in turn, 31 / 67 / 347 us with a lane per pair and a wave per
+// 16 tiles, 20 / 56 / 146 us with the even split (the larger ones beside the interior kernel),
+// 20 / 30 / 82 us in turn with it.
 //
 // Neighbouring silhouette pairs share vertices: a wave takes 64 pairs at a time, a pair stores
 // its 8 entries (two triangles' corners, the window gradients of the edge's ends), each rounded

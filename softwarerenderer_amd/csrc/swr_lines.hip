@@ -210,7 +210,7 @@ __device__ inline void write_fragment(const LineArgs &A, uint64_t f, uint64_t i,
 // all lanes in pieces, line by line, so that a wave takes as long as its lines together and not
 // as its longest.  Bound by the serial steps of a piece (and in the emit pass by its scattered
 // record stores): 60,000 lines, a fifth of them across a 1920x1080 screen, took 269 us to count
-// and 656 us to emit with a thread per line, now 122 and 374 us (195 and 453 us with 64 lines per
+// and 656 us to emit with a thread per line, now 117 and 374 us (195 and 453 us with 64 lines per
 // wave, which leaves too few waves); 60,000 points 48 us to count with the totals as atomics on
 // two words, now 6 us.
 constexpr uint32_t LINE_PIECE = 32, LINES = 16;

@@ -24,14 +24,17 @@
 // the registers' sake) the 8 slots hold several planes of each.  Phase B: lane = pixel shades
 // the GS primitives in draw order.
 //
-// What bounds it: VALU issue (88% of it on dense frames before the steps below).  Per group
-// of 8 primitives the row starts cost 7 DPP additions per chain (14 instructions as additions
-// and selects), programs that only test z take no coverage masks (NaN rows), coverage of
-// every kind is three stepped compares without branches, a group's record loads leave
-// together, and larger bins drop hidden primitives of long lists for programs that only test
-// z.  1080p soup of 1M triangles, Block, 16-pixel bins: 109 -> 74 us; 150k triangles,
-// Adaptive, 1003x701: 87 -> 80 us; 10-plane hash program on 12.7M pairs: 4699 us with half
-// the slots idle, 3237 us with two planes per primitive in them.
+// What bounds it: vector issue and the wait for loads, about evenly.  On the 1080p soup of 1M
+// triangles it issues 609 G wave instructions/s (plain additions reach 1020 here, compares, fp64
+// and 32-bit products 575), and a wave spends 41% of its time waiting for results, 31% ready and
+// waiting for issue, 28% issuing; the hash program's longest lists leave the CUs busy for 58% of
+// the launch.  Per group of 8 primitives the row starts cost 7 DPP additions per chain (14
+// instructions as additions and selects), programs that only test z take no coverage masks (NaN
+// rows), coverage of every kind is three stepped compares without branches, a group's record
+// loads leave together, and larger bins drop hidden primitives of long lists for programs that
+// only test z.  1080p soup of 1M triangles, Block, 16-pixel bins: 109 -> 75 us; 150k triangles,
+// Adaptive, 1003x701: 87 -> 69 us; 10-plane hash program on 12.7M pairs: 4699 us with half
+// the slots idle, 3239 us with two planes per primitive in them.
 //
 // The kernel is a template over the pixel program, so that programs compiled outside the
 // library (include/swr/pixel_program.h) instantiate it the same way the built-in ones do.

@@ -536,7 +536,8 @@ static uint32_t fan_blocks(uint64_t batches)
 size_t fan_scan_bytes(uint64_t batches) { return ((size_t)fan_blocks(batches) + 1) * 16; }
 
 // Draws of up to this many workgroups (16k triangles) take one launch: adding up what lies
-// before costs a workgroup at most 48 KB of reads that hit the L2, a launch some 5 us.
+// before costs the last workgroup 60 KB of reads that hit the L2 (5 bytes for each of 12,288
+// triangles; at most 96 KB more where clipping appends fans), a launch some 5 us.
 constexpr uint32_t FAN_ONE_PASS = 4;
 
 hipError_t scan_fans(const uint32_t *cnt, const uint8_t *cflag, const uint2 *app, uint2 *ex,

@@ -6,8 +6,8 @@ Forward, for V views of one triangle mesh:
      program: nearest source triangle + 1 and its depth per pixel);
   2. ``swr_diff_forward``: perspective-correct barycentrics, the interpolated attributes and
      the analytic edge-antialiasing blend across silhouette edges.
-Backward: ``swr_diff_backward`` recomputes everything it needs from the visibility buffer,
-the barycentrics and the colour, and returns d(loss)/d(clip positions) per view and
+Backward: ``swr_diff_backward`` recomputes everything it needs from the visibility buffer, the
+clip positions and the attributes, and returns d(loss)/d(clip positions) per view and
 d(loss)/d(attributes).  Gradients w.r.t. world-space positions follow through torch's
 own autograd of the projection that produced the clip positions.
 
